@@ -1,205 +1,250 @@
-// fp32 backward of the attention output (gfx950, VALU): the reference's
+// fp32 backward of the attention output (gfx950, fp32 MFMA): the reference's
 // algorithm (fused_self_attention.cpp:66-135) in the same two passes and with
-// the same workspace as the 16-bit kernels (attn_bwd_kernels.hpp), on the
-// vector ALUs.  The float path serves the reference's own float
-// configuration (small, launch-bound shapes), so it is written for clarity:
-// one wave per owned row, four waves per workgroup.
+// the same workspace as the 16-bit kernels (attn_bwd_kernels.hpp).
 //
-//   attn_bwd_f32_dq_kernel    wave = query row i.  Lane = key j within a chunk
-//                             of 64 for s_ij = <q_i, k_j> and dP_ij =
-//                             <dout_i, v_j> (q_i and dout_i spread over the
-//                             lanes by head_dim element and broadcast with
-//                             readlane), then lane = head_dim element for
-//                             dq_i += dS_ij k_j, dS_ij taken lane by lane.
+//   attn_bwd_f32_dq_kernel    a workgroup owns 32 query rows; its four waves
+//                             take the key tiles (of 32) w, w + 4, ... .  Per
+//                             tile dP^T = V dout^T and S^T = K Q^T, then P and
+//                             dS in the accumulator registers, which are the B
+//                             operand of dQ^T += K^T dS^T as they stand.
 //                             Writes lse2_i and D_i to the workspace.
-//   attn_bwd_f32_dkdv_kernel  wave = key row j, lane = query i in a chunk of
-//                             64 for s_ij, dP_ij, P_ij = exp2(s_ij c - lse2_i)
-//                             and dS_ij = P_ij (dP_ij - D_i); then lane =
-//                             head_dim element for dv_j += P_ij dout_i and
-//                             dk_j += dS_ij q_i.
+//   attn_bwd_f32_dkdv_kernel  a workgroup owns 32 key rows, its waves split
+//                             the query tiles: dP = dout V^T, S = Q K^T,
+//                             dK^T += Q^T dS, dV^T += dout^T P.
+//
+// Bound: v_mfma_f32_32x32x2f32 (attn_f32.hpp).  Each wave stages its own
+// tiles, V then K (dout, Q, dout) through one LDS tile and one set of staging
+// registers, the next one in flight under the products of the one before: the
+// waves of a SIMD (4 / 3 / 1 at head_dim 32 / 64 / 128) drift apart and one's
+// exponentials and LDS writes pass under the other's MFMAs.  32 owned rows and
+// a four-way split give many short, equal workgroups: the chains of dependent
+// tiles are a quarter as long as with one wave per row block, which bounds the
+// small shapes, and the long causal rows start first.
+// Measured against one wave per owned row on the vector ALUs (dq / dkdv, us):
+// B4 H16 S1024 D64 causal 3,141 / 3,303 -> 132 / 180 (96 and 128 fp32 MFMAs per
+// tile: 84 and 112 us at the MFMA's 154 TFLOP/s), B2 H16 S128 D128 90 / 123 ->
+// 14 / 16 (one tile per wave: latency).
 #pragma once
 
 #include "attn_bwd_kernels.hpp"
+#include "attn_f32.hpp"
 
 namespace pmkl_amd {
 
-constexpr int kBwdF32Waves = 4;   // owned rows per workgroup (one per wave)
-
-__device__ __forceinline__ float bwd_f32_wave_sum(float x) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) x += __shfl_xor(x, o, 64);
-    return x;
-}
-
-// Value of lane `src` (uniform) of x.
-__device__ __forceinline__ float bwd_f32_lane(float x, int src) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), src));
-}
-
-// <a, row>: a[d] is held by lane d % 64 in register a[d / 64]; row is this
-// lane's own 16-byte aligned row of D floats.
-template <int D>
-__device__ __forceinline__ float bwd_f32_dot(const float (&a)[(D + 63) / 64], const float *row) {
-    float acc = 0.f;
-#pragma unroll
-    for (int d = 0; d < D; d += 4) {
-        const f32x4_t r = *(const f32x4_t *)(row + d);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc = __builtin_fmaf(bwd_f32_lane(a[(d + e) / 64], (d + e) % 64), r[e], acc);
-    }
-    return acc;
-}
-
 template <int D, bool CAUSAL>
-__global__ __launch_bounds__(kBwdF32Waves * 64) void attn_bwd_f32_dq_kernel(BwdParams p) {
-    constexpr int NE = (D + 63) / 64;   // head_dim elements per lane
-    const int lane = threadIdx.x & 63;
-    const int S = p.S;
-    const int64_t row = (int64_t)blockIdx.x * kBwdF32Waves + (threadIdx.x >> 6);   // bh * S + qi
-    if (row >= (int64_t)p.BH * S) return;   // the whole wave
-    const int64_t bh = row / S;
-    const int qi = (int)(row - bh * S);
-    const float *kg = bwd_head<const float>(p, p.k, BK, (int)bh);
-    const float *vg = bwd_head<const float>(p, p.v, BV, (int)bh);
-    const int kss = p.ss[BK], vss = p.ss[BV];
-    const float *qr_i = bwd_head<const float>(p, p.q, BQ, (int)bh) + (int64_t)qi * p.ss[BQ];
-    const float *dr_i = bwd_head<const float>(p, p.dout, BDOUT, (int)bh) + (int64_t)qi * p.ss[BDOUT];
+__global__ __launch_bounds__(kF32Threads, D >= 128 ? 1 : D >= 64 ? 3 : 4) void attn_bwd_f32_dq_kernel(BwdParams p) {
+    using TL = F32Tile<D>;
+    constexpr int NW = kF32Waves, BN = kF32Rows, NDB = D / 32;
+    __shared__ __attribute__((aligned(16))) float smem[NW][TL::FLOATS];   // each wave's V or K tile
+    __shared__ __attribute__((aligned(16))) float dtile[TL::FLOATS];      // dout of the owned rows
+    __shared__ float dvec[NW][BN];   // D_i, or each wave's part of it
 
-    float qv[NE], dov[NE];
-#pragma unroll
-    for (int e = 0; e < NE; ++e) {
-        const int d = lane + 64 * e;
-        qv[e] = d < D ? qr_i[d] : 0.f;
-        dov[e] = d < D ? dr_i[d] : 0.f;
-    }
-    const float m_i = bwd_load_ml<float>(p.m, row, true);
-    const float l_i = bwd_load_ml<float>(p.l, row, true);
+    const int lane = threadIdx.x & 63;
+    const int hi = lane >> 5, col = lane & 31;
+    const int bh = blockIdx.x % p.BH;
+    const int qt = CAUSAL ? p.n_qtiles - 1 - (int)blockIdx.x / p.BH : (int)blockIdx.x / p.BH;   // longest first
+    const int wave = f32_wave(bh, qt);
+    const int S = p.S;
+    const float *kg = bwd_head<const float>(p, p.k, BK, bh);
+    const float *vg = bwd_head<const float>(p, p.v, BV, bh);
+    const int kss = p.ss[BK], vss = p.ss[BV];
+    const int q0 = qt * BN;
+    const int qi = q0 + col;                  // this lane's query row
+    const int qrow = min(qi, S - 1);
+    const int lim = CAUSAL ? qrow : S - 1;    // its last visible key
+    const int nt = (CAUSAL ? min(q0 + BN - 1, S - 1) : S - 1) / BN + 1;
+
+    float *tile = smem[wave];
+    F32Stage<D, 64> st;
+    auto load_v = [&](int kt) __attribute__((always_inline)) { st.load(vg, kt * BN, kt < nt ? S : 0, vss, lane); };
+
+    // The owned rows, loaded once by the whole workgroup and handed to the
+    // waves through LDS; D_i = <dout_i, o_i> from the same
+    // loads where the caller passes O.
+    F32Stage<D, kF32Threads> qst, dst, ost;
+    qst.load(bwd_head<const float>(p, p.q, BQ, bh), q0, S, p.ss[BQ], threadIdx.x);
+    dst.load(bwd_head<const float>(p, p.dout, BDOUT, bh), q0, S, p.ss[BDOUT], threadIdx.x);
+    if (p.o != nullptr) ost.load(bwd_head<const float>(p, p.o, BO, bh), q0, S, p.ss[BO], threadIdx.x);
+    const float m_i = bwd_load_ml<float>(p.m, (int64_t)bh * S + qrow, true);
+    const float l_i = bwd_load_ml<float>(p.l, (int64_t)bh * S + qrow, true);
+    load_v(wave);
     const float lse2 = m_i * 1.4426950408889634f + __log2f(l_i);
     const float c = p.scale_log2;
-    const int last = CAUSAL ? qi : S - 1;   // last visible key
+    qst.store(smem[0], threadIdx.x);
+    dst.store(dtile, threadIdx.x);
+    if (p.o != nullptr) {
+#pragma unroll
+        for (int j = 0; j < decltype(ost)::LOADS; ++j) {
+            float part = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part = __builtin_fmaf(ost.reg[j][e], dst.reg[j][e], part);
+#pragma unroll
+            for (int o = TL::CPR / 2; o >= 1; o >>= 1) part += __shfl_xor(part, o, 64);   // the row's chunks
+            if (threadIdx.x % TL::CPR == 0) dvec[0][threadIdx.x / TL::CPR + j * decltype(ost)::STEP] = part;
+        }
+    }
+    __syncthreads();
+    f32x4_t qf[D / 8];
+    f32_rows<D>(qf, smem[0], col, hi);
+    float drow = p.o != nullptr ? dvec[0][col] : 0.f;
+    __syncthreads();
 
-    // P and dP of this lane's key j0 + lane (0 past the last visible key)
-    auto prob = [&](int j0, float &pv, float &dp) __attribute__((always_inline)) {
-        const int j = j0 + lane;
-        const int jc = j <= last ? j : last;
-        const float s = bwd_f32_dot<D>(qv, kg + (int64_t)jc * kss);
-        dp = bwd_f32_dot<D>(dov, vg + (int64_t)jc * vss);
-        pv = j <= last ? fast_exp2(__builtin_fmaf(s, c, -lse2)) : 0.f;
+    // This wave's tiles; work(P, dP) gets the probabilities and dP of a tile.
+    // The wave's own LDS: its reads of the previous tile are issued before
+    // the writes of the next, and one wave's LDS operations run in order, so
+    // neither side needs a barrier.  On return the first tile is in flight
+    // again where another loop follows.
+    auto tiles = [&](auto last_c, auto &&work) __attribute__((always_inline)) {
+        for (int kt = wave; kt < nt; kt += NW) {
+            asm volatile("" ::: "memory");
+            st.store(tile, lane);
+            asm volatile("" ::: "memory");
+            st.load(kg, kt * BN, S, kss, lane);
+            f32x16_t s{}, dp{};
+            f32_scores<D>(tile, dtile, dp, col, hi);
+            asm volatile("" ::: "memory");
+            st.store(tile, lane);
+            asm volatile("" ::: "memory");
+            load_v(decltype(last_c)::value || kt + NW < nt ? kt + NW : wave);
+            f32_scores<D>(tile, qf, s, col, hi);
+            const int d = lim - kt * BN - 4 * hi;   // f32_acc_row up to d is visible
+            if (kt * BN + BN - 1 > (CAUSAL ? q0 : S - 1)) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    s[r] = f32_acc_row(r) <= d ? fast_exp2(__builtin_fmaf(s[r], c, -lse2)) : 0.f;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[r] = fast_exp2(__builtin_fmaf(s[r], c, -lse2));
+            }
+            work(s, dp);
+        }
     };
 
-    float drow;
-    if (p.o != nullptr) {
-        const float *or_i = bwd_head<const float>(p, p.o, BO, (int)bh) + (int64_t)qi * p.ss[BO];
+    if (p.o == nullptr) {   // D_i = sum_j P_ij dP_ij over the keys
         float part = 0.f;
+        tiles(std::false_type{}, [&](const f32x16_t &pr, const f32x16_t &dp) __attribute__((always_inline)) {
 #pragma unroll
-        for (int e = 0; e < NE; ++e) {
-            const int d = lane + 64 * e;
-            if (d < D) part = __builtin_fmaf(or_i[d], dov[e], part);
-        }
-        drow = bwd_f32_wave_sum(part);
-    } else {
-        float part = 0.f;
-        for (int j0 = 0; j0 <= last; j0 += 64) {
-            float pv, dp;
-            prob(j0, pv, dp);
-            part = __builtin_fmaf(pv, dp, part);
-        }
-        drow = bwd_f32_wave_sum(part);
+            for (int r = 0; r < 16; ++r) part = __builtin_fmaf(pr[r], dp[r], part);
+        });
+        part = half_sum(part);
+        if (hi == 0) dvec[wave][col] = part;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < NW; ++w) drow += dvec[w][col];   // waves without tiles wrote 0
     }
-    if (lane == 0) {
-        p.lse2[row] = lse2;
-        p.drow[row] = drow;
+    if (wave == 0 && hi == 0 && qi < S) {
+        p.lse2[(int64_t)bh * S + qi] = lse2;
+        p.drow[(int64_t)bh * S + qi] = drow;
     }
 
-    float acc[NE];
+    f32x16_t acc[NDB];   // dQ^T (head_dim x owned rows), this wave's tiles
 #pragma unroll
-    for (int e = 0; e < NE; ++e) acc[e] = 0.f;
-    for (int j0 = 0; j0 <= last; j0 += 64) {
-        float pv, dp;
-        prob(j0, pv, dp);
-        const float ds = pv * (dp - drow);
-        const int n = min(64, last - j0 + 1);
-        for (int jj = 0; jj < n; ++jj) {
-            const float dsj = bwd_f32_lane(ds, jj);
-            const float *kr = kg + (int64_t)(j0 + jj) * kss;
+    for (int db = 0; db < NDB; ++db) acc[db] = f32x16_t{};
+    tiles(std::true_type{}, [&](f32x16_t &pr, const f32x16_t &dp) __attribute__((always_inline)) {
 #pragma unroll
-            for (int e = 0; e < NE; ++e) {
-                const int d = lane + 64 * e;
-                if (d < D) acc[e] = __builtin_fmaf(dsj, kr[d], acc[e]);
-            }
-        }
-    }
-    float *dq_i = bwd_head<float>(p, p.dq, BDQ, (int)bh) + (int64_t)qi * p.ss[BDQ];
-#pragma unroll
-    for (int e = 0; e < NE; ++e) {
-        const int d = lane + 64 * e;
-        if (d < D) dq_i[d] = acc[e] * p.scale;
-    }
+        for (int r = 0; r < 16; ++r) pr[r] *= dp[r] - drow;   // dS
+        f32_accumulate<D>(tile, pr, acc, col, hi);
+    });
+
+    asm volatile("" ::: "memory");
+    if (wave < nt) f32_put<D>(tile, acc, col, hi);
+    __syncthreads();
+    f32_combine<D>(smem[0], TL::FLOATS, min(NW, nt), p.scale, bwd_head<float>(p, p.dq, BDQ, bh), q0, S,
+                       p.ss[BDQ]);
 }
 
 template <int D, bool CAUSAL>
-__global__ __launch_bounds__(kBwdF32Waves * 64) void attn_bwd_f32_dkdv_kernel(BwdParams p) {
-    constexpr int NE = (D + 63) / 64;
-    const int lane = threadIdx.x & 63;
-    const int S = p.S;
-    const int64_t row = (int64_t)blockIdx.x * kBwdF32Waves + (threadIdx.x >> 6);   // bh * S + kj
-    if (row >= (int64_t)p.BH * S) return;
-    const int64_t bh = row / S;
-    const int kj = (int)(row - bh * S);
-    const float *qg = bwd_head<const float>(p, p.q, BQ, (int)bh);
-    const float *dog = bwd_head<const float>(p, p.dout, BDOUT, (int)bh);
-    const int qss = p.ss[BQ], doss = p.ss[BDOUT];
-    const float *lse2g = p.lse2 + bh * S;
-    const float *drowg = p.drow + bh * S;
-    const float *kr_j = bwd_head<const float>(p, p.k, BK, (int)bh) + (int64_t)kj * p.ss[BK];
-    const float *vr_j = bwd_head<const float>(p, p.v, BV, (int)bh) + (int64_t)kj * p.ss[BV];
+__global__ __launch_bounds__(kF32Threads, D >= 128 ? 1 : D >= 64 ? 3 : 4) void attn_bwd_f32_dkdv_kernel(BwdParams p) {
+    using TL = F32Tile<D>;
+    constexpr int NW = kF32Waves, BN = kF32Rows, NDB = D / 32;
+    __shared__ __attribute__((aligned(16))) float smem[NW][TL::FLOATS];   // each wave's dout or Q tile
+    __shared__ __attribute__((aligned(16))) float own[2][TL::FLOATS];     // the owned K and V rows
+    __shared__ __attribute__((aligned(16))) float svec[NW][2][BN];        // lse2, D_i of its rows
 
-    float kv[NE], vv[NE];
-#pragma unroll
-    for (int e = 0; e < NE; ++e) {
-        const int d = lane + 64 * e;
-        kv[e] = d < D ? kr_j[d] : 0.f;
-        vv[e] = d < D ? vr_j[d] : 0.f;
+    const int lane = threadIdx.x & 63;
+    const int hi = lane >> 5, col = lane & 31;
+    const int bh = blockIdx.x % p.BH;
+    const int kt = (int)blockIdx.x / p.BH;   // the first keys have the most queries (causal)
+    const int wave = f32_wave(bh, kt);
+    const int S = p.S;
+    const float *qg = bwd_head<const float>(p, p.q, BQ, bh);
+    const float *dog = bwd_head<const float>(p, p.dout, BDOUT, bh);
+    const int qss = p.ss[BQ], doss = p.ss[BDOUT];
+    const int k0 = kt * BN;
+    const int kj = k0 + col;                 // this lane's key row
+    const int t0 = CAUSAL ? kt : 0;          // first query tile with a visible query
+    const int nq = (S - 1) / BN + 1;
+
+    float *tile = smem[wave], *vec = svec[wave][0];
+    F32Stage<D, 64> st;
+    float vreg;   // lanes 0-31: lse2, 32-63: D_i of the tile's rows
+    const float *vecg = (hi ? p.drow : p.lse2) + (int64_t)bh * S;
+    auto load_do = [&](int t) __attribute__((always_inline)) { st.load(dog, t * BN, t < nq ? S : 0, doss, lane); };
+    auto load_vec = [&](int t) __attribute__((always_inline)) {
+        // rows past S: lse2 = +inf and zero Q, dout rows give P = 0, dS = 0
+        vreg = t * BN + col < S ? vecg[t * BN + col] : (hi ? 0.f : INFINITY);
+    };
+
+    {
+        F32Stage<D, kF32Threads> kst, vst;
+        kst.load(bwd_head<const float>(p, p.k, BK, bh), k0, S, p.ss[BK], threadIdx.x);
+        vst.load(bwd_head<const float>(p, p.v, BV, bh), k0, S, p.ss[BV], threadIdx.x);
+        load_do(t0 + wave);
+        load_vec(t0 + wave);
+        kst.store(own[0], threadIdx.x);
+        vst.store(own[1], threadIdx.x);
+        __syncthreads();
     }
     const float c = p.scale_log2;
-    const int first = CAUSAL ? kj : 0;   // first query that sees key kj
 
-    float acc_k[NE], acc_v[NE];
+    f32x16_t dk_acc[NDB], dv_acc[NDB];   // dK^T, dV^T (head_dim x owned keys), this wave's tiles
 #pragma unroll
-    for (int e = 0; e < NE; ++e) acc_k[e] = acc_v[e] = 0.f;
-    for (int i0 = first; i0 < S; i0 += 64) {
-        const int i = i0 + lane;
-        const int ic = i < S ? i : S - 1;
-        const float s = bwd_f32_dot<D>(kv, qg + (int64_t)ic * qss);
-        const float dp = bwd_f32_dot<D>(vv, dog + (int64_t)ic * doss);
-        const float pv = i < S ? fast_exp2(__builtin_fmaf(s, c, -lse2g[ic])) : 0.f;
-        const float ds = pv * (dp - drowg[ic]);
-        const int n = min(64, S - i0);
-        for (int ii = 0; ii < n; ++ii) {
-            const float pi = bwd_f32_lane(pv, ii);
-            const float dsi = bwd_f32_lane(ds, ii);
-            const float *qr = qg + (int64_t)(i0 + ii) * qss;
-            const float *dr = dog + (int64_t)(i0 + ii) * doss;
+    for (int db = 0; db < NDB; ++db) dk_acc[db] = dv_acc[db] = f32x16_t{};
+    for (int t = t0 + wave; t < nq; t += NW) {
+        asm volatile("" ::: "memory");
+        st.store(tile, lane);
+        vec[lane] = vreg;
+        asm volatile("" ::: "memory");
+        st.load(qg, t * BN, S, qss, lane);
+        load_vec(t + NW);
+        f32x16_t s{}, dp{};
+        f32_scores<D>(tile, own[1], dp, col, hi);
+        asm volatile("" ::: "memory");
+        st.store(tile, lane);
+        asm volatile("" ::: "memory");
+        load_do(t);
+        f32_scores<D>(tile, own[0], s, col, hi);
+        const int d = kj - t * BN - 4 * hi;   // causal: f32_acc_row from d on sees the key
+        const bool mask = CAUSAL && t == t0;
 #pragma unroll
-            for (int e = 0; e < NE; ++e) {
-                const int d = lane + 64 * e;
-                if (d < D) {
-                    acc_v[e] = __builtin_fmaf(pi, dr[d], acc_v[e]);
-                    acc_k[e] = __builtin_fmaf(dsi, qr[d], acc_k[e]);
-                }
+        for (int g = 0; g < 4; ++g) {
+            const f32x4_t l4 = *(const f32x4_t *)(vec + 8 * g + 4 * hi), d4 = *(const f32x4_t *)(vec + BN + 8 * g + 4 * hi);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int r = 4 * g + e;
+                const float pv = fast_exp2(__builtin_fmaf(s[r], c, -l4[e]));
+                s[r] = !mask || f32_acc_row(r) >= d ? pv : 0.f;
+                dp[r] = s[r] * (dp[r] - d4[e]);
             }
         }
+        f32_accumulate<D>(tile, dp, dk_acc, col, hi);
+        asm volatile("" ::: "memory");
+        st.store(tile, lane);
+        asm volatile("" ::: "memory");
+        load_do(t + NW);
+        f32_accumulate<D>(tile, s, dv_acc, col, hi);
     }
-    float *dk_j = bwd_head<float>(p, p.dk, BDK, (int)bh) + (int64_t)kj * p.ss[BDK];
-    float *dv_j = bwd_head<float>(p, p.dv, BDV, (int)bh) + (int64_t)kj * p.ss[BDV];
-#pragma unroll
-    for (int e = 0; e < NE; ++e) {
-        const int d = lane + 64 * e;
-        if (d < D) {
-            dk_j[d] = acc_k[e] * p.scale;
-            dv_j[d] = acc_v[e];
-        }
-    }
+
+    // dK, then dV, through the waves' tiles
+    const int n = min(NW, nq - t0);
+    asm volatile("" ::: "memory");
+    if (t0 + wave < nq) f32_put<D>(tile, dk_acc, col, hi);
+    __syncthreads();
+    f32_combine<D>(smem[0], TL::FLOATS, n, p.scale, bwd_head<float>(p, p.dk, BDK, bh), k0, S, p.ss[BDK]);
+    __syncthreads();
+    if (t0 + wave < nq) f32_put<D>(tile, dv_acc, col, hi);
+    __syncthreads();
+    f32_combine<D>(smem[0], TL::FLOATS, n, 1.f, bwd_head<float>(p, p.dv, BDV, bh), k0, S, p.ss[BDV]);
 }
 
 }  // namespace pmkl_amd

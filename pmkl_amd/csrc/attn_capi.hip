@@ -295,7 +295,6 @@ struct BwdKernels {
     bwd_kernel_fn dq, dkdv;
     int dq_threads, dq_rows;       // threads and owned rows per workgroup
     int dkdv_threads, dkdv_rows;
-    bool flat;                     // grid over the B*H*S rows, else (row tile, head)
 };
 
 template <typename T, int D>
@@ -304,19 +303,17 @@ BwdKernels pick_bwd(bool causal) {
     using TK = pmkl_amd::BwdTile<T, D, pmkl_amd::bwd_waves_dkdv<D>()>;
     if (causal)
         return {pmkl_amd::attn_bwd_dq_kernel<T, D, true>, pmkl_amd::attn_bwd_dkdv_kernel<T, D, true>, TQ::THREADS,
-                TQ::ROWS, TK::THREADS, TK::ROWS, false};
+                TQ::ROWS, TK::THREADS, TK::ROWS};
     return {pmkl_amd::attn_bwd_dq_kernel<T, D, false>, pmkl_amd::attn_bwd_dkdv_kernel<T, D, false>, TQ::THREADS,
-            TQ::ROWS, TK::THREADS, TK::ROWS, false};
+            TQ::ROWS, TK::THREADS, TK::ROWS};
 }
 
 template <int D>
 BwdKernels pick_bwd_f32(bool causal) {
-    constexpr int W = pmkl_amd::kBwdF32Waves;
+    constexpr int T = pmkl_amd::kF32Threads, R = pmkl_amd::kF32Rows;
     if (causal)
-        return {pmkl_amd::attn_bwd_f32_dq_kernel<D, true>, pmkl_amd::attn_bwd_f32_dkdv_kernel<D, true>, 64 * W, W,
-                64 * W, W, true};
-    return {pmkl_amd::attn_bwd_f32_dq_kernel<D, false>, pmkl_amd::attn_bwd_f32_dkdv_kernel<D, false>, 64 * W, W,
-            64 * W, W, true};
+        return {pmkl_amd::attn_bwd_f32_dq_kernel<D, true>, pmkl_amd::attn_bwd_f32_dkdv_kernel<D, true>, T, R, T, R};
+    return {pmkl_amd::attn_bwd_f32_dq_kernel<D, false>, pmkl_amd::attn_bwd_f32_dkdv_kernel<D, false>, T, R, T, R};
 }
 
 BwdKernels select_bwd(int32_t dt, int64_t d, bool causal) {
@@ -333,7 +330,7 @@ BwdKernels select_bwd(int32_t dt, int64_t d, bool causal) {
         if (d == 64) return pick_bwd_f32<64>(causal);
         if (d == 128) return pick_bwd_f32<128>(causal);
     }
-    return {nullptr, nullptr, 0, 0, 0, 0, false};
+    return {nullptr, nullptr, 0, 0, 0, 0};
 }
 
 // One [B, H, S, D] tensor of a backward call, for the checks and the launch.
@@ -388,8 +385,7 @@ int check_bwd(const pmkl_attn_bwd_args *a, bool *empty) {
     PMKL_REQUIRE(kc.dq != nullptr, PMKL_EUNSUPPORTED, "no backward kernel for dtype %d head_dim %lld",
                  (int)a->dtype, (long long)D);
     const int64_t nq = (S + kc.dq_rows - 1) / kc.dq_rows, nk = (S + kc.dkdv_rows - 1) / kc.dkdv_rows;
-    const int64_t gq = kc.flat ? (B * H * S + kc.dq_rows - 1) / kc.dq_rows : nq * B * H;
-    const int64_t gk = kc.flat ? (B * H * S + kc.dkdv_rows - 1) / kc.dkdv_rows : nk * B * H;
+    const int64_t gq = nq * B * H, gk = nk * B * H;
     PMKL_REQUIRE(std::max(gq, gk) <= 0x7fffffffLL, PMKL_EINVAL, "grid too large (%lld workgroups)",
                  (long long)std::max(gq, gk));
     return PMKL_OK;
@@ -403,8 +399,7 @@ int launch_bwd(const pmkl_attn_bwd_args *a, float *ws, void *stream) {
     const int64_t B = a->batch, H = a->heads, S = a->seq_len, D = a->head_dim;
     const BwdKernels kc = select_bwd(a->dtype, D, a->is_causal != 0);
     const int64_t nq = (S + kc.dq_rows - 1) / kc.dq_rows, nk = (S + kc.dkdv_rows - 1) / kc.dkdv_rows;
-    const int64_t gq = kc.flat ? (B * H * S + kc.dq_rows - 1) / kc.dq_rows : nq * B * H;
-    const int64_t gk = kc.flat ? (B * H * S + kc.dkdv_rows - 1) / kc.dkdv_rows : nk * B * H;
+    const int64_t gq = nq * B * H, gk = nk * B * H;
 
     BwdParams p;
     p.q = a->q;
