@@ -25,6 +25,7 @@
 #include "attn_fwd_w64.hpp"
 #include "attn_bwd_kernels.hpp"
 #include "attn_bwd_f32.hpp"
+#include "attn_fwd_f32.hpp"
 
 // The 64-row forward kernels are instantiated in attn_fwd_w64_<dtype>_<mask>.hip
 // (one translation unit each, compiled in parallel).
@@ -163,8 +164,7 @@ bool split_enabled() {
     }();
     return on;
 }
-// fp32 problems too small to fill the CUs take the key-split kernel unless
-// PMKL_ATTN_F32SPLIT=0 (read once).
+// fp32 takes the key-split kernel unless PMKL_ATTN_F32SPLIT=0 (read once).
 bool f32split_enabled() {
     static const bool on = [] {
         const char *e = getenv("PMKL_ATTN_F32SPLIT");
@@ -552,10 +552,12 @@ int plan_fwd(const pmkl_attn_fwd_args *a, FwdPlan *pl) {
                           (S + 63) / 64 <= resident_tiles(D) && resident_enabled();
     const bool split = w32 && D == 64 && causal && split_enabled() &&
                        B * H * ((S + 255) / 256) < 2 * (int64_t)cu_count();
-    // fp32 with the 128-row kernel's workgroups on fewer than half the CUs
-    // (C1: 4): 32-row workgroups whose four waves split the key tiles.
-    const bool f32split = a->dtype == PMKL_DTYPE_F32 && f32split_enabled() && S <= 1024 &&
-                          B * H * ((S + 127) / 128) * 2 < (int64_t)cu_count();
+    // fp32: 32-row workgroups whose four waves split the key tiles, at every
+    // size (measured against the 128-row kernel, us: B1 H4 S128 D64 6.3 / 17.1,
+    // B4 H16 S1024 D64 96 / 126, B2 H4 S2048 D128 144 / 326, B1 H32 S4096 D128
+    // 1,109 / 1,357, B256 H8 S20 D64 19.1 / 21.4).  The 128-row kernel is left
+    // for PMKL_ATTN_F32SPLIT=0 and for a device whose CU count cannot be read.
+    const bool f32split = a->dtype == PMKL_DTYPE_F32 && f32split_enabled() && cu_count() > 0;
     const KernelChoice kc = w32        ? (bf ? pick_w32<__bf16>(D, causal, split) : pick_w32<_Float16>(D, causal, split))
                             : f32split ? pick32split(D, causal)
                                        : select_kernel(a->dtype, D, causal, w64, waves, resident);
