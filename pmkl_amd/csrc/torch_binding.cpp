@@ -224,6 +224,76 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> fused_self_attention_fw(const at:
     return std::forward_as_tuple(out, out_m, out_l);
 }
 
+namespace {
+
+// Device backward; out (the forward's output) may be undefined.
+std::tuple<at::Tensor, at::Tensor, at::Tensor> device_backward(const at::Tensor &dout, const at::Tensor &q,
+                                                               const at::Tensor &k, const at::Tensor &v,
+                                                               const at::Tensor &out, const at::Tensor &out_m,
+                                                               const at::Tensor &out_l, bool is_causal) {
+    const int64_t B = q.size(0), H = q.size(1), S = q.size(2), D = q.size(3);
+    const int32_t dt = to_pmkl_dtype(q.scalar_type());
+    TORCH_CHECK(pmkl_attn_bwd_supported(dt, D), "fused_self_attention_bw: the device backward supports float32, ",
+                "float16 and bfloat16 with head_dim 32, 64 or 128, got ", q.scalar_type(), " head_dim ", D);
+    // Gradients come back contiguous [B, H, S, D]; the kernels write every element.
+    auto gopts = q.options().memory_format(at::MemoryFormat::Contiguous);
+    auto dq = at::empty({B, H, S, D}, gopts);
+    auto dk = at::empty({B, H, S, D}, gopts);
+    auto dv = at::empty({B, H, S, D}, gopts);
+    if (B * H * S == 0) return std::forward_as_tuple(dq, dk, dv);
+    const int32_t mdt = to_pmkl_dtype(out_m.scalar_type());
+    TORCH_CHECK(out_m.scalar_type() == out_l.scalar_type() && (mdt == dt || mdt == PMKL_DTYPE_F32),
+                "fused_self_attention_bw: out_m / out_l must be in the tensors' dtype or float32");
+
+    c10::OptionalDeviceGuard guard(q.device());
+    auto mc = out_m.contiguous(), lc = out_l.contiguous();
+    // Strided views go to the kernels as they are; only a layout the kernels
+    // cannot address (head_dim not contiguous, strides or base not 16-byte
+    // aligned) is copied.
+    auto qd = device_view(q), kd = device_view(k), vd = device_view(v), dod = device_view(dout);
+    auto od = out.defined() ? device_view(out) : at::Tensor();
+    const uint64_t ws_bytes = pmkl_attn_bwd_workspace_size(B, H, S);
+    auto ws = at::empty({(int64_t)((ws_bytes + 3) / 4)}, q.options().dtype(at::kFloat));
+    pmkl_attn_bwd_args a;
+    std::memset(&a, 0, sizeof(a));
+    a.dout = dod.data_ptr();
+    a.q = qd.data_ptr();
+    a.k = kd.data_ptr();
+    a.v = vd.data_ptr();
+    fill_strides(a.dout_strides, dod);
+    fill_strides(a.q_strides, qd);
+    fill_strides(a.k_strides, kd);
+    fill_strides(a.v_strides, vd);
+    fill_strides(a.dq_strides, dq);
+    fill_strides(a.dk_strides, dk);
+    fill_strides(a.dv_strides, dv);
+    if (od.defined()) {
+        a.o = od.data_ptr();
+        fill_strides(a.o_strides, od);
+    }
+    a.m = mc.data_ptr();
+    a.l = lc.data_ptr();
+    a.dq = dq.data_ptr();
+    a.dk = dk.data_ptr();
+    a.dv = dv.data_ptr();
+    a.workspace = ws.data_ptr();
+    a.workspace_bytes = (uint64_t)ws.numel() * 4;
+    a.dtype = dt;
+    a.ml_dtype = mdt;
+    a.batch = B;
+    a.heads = H;
+    a.seq_len = S;
+    a.head_dim = D;
+    a.scale = 0.f;
+    a.is_causal = is_causal ? 1 : 0;
+    hipStream_t stream = c10::hip::getCurrentHIPStream(q.device().index()).stream();
+    const int rc = pmkl_attn_bwd(&a, (void *)stream);
+    TORCH_CHECK(rc == PMKL_OK, "fused_self_attention_bw: ", pmkl_last_error());
+    return std::forward_as_tuple(dq, dk, dv);
+}
+
+}  // namespace
+
 std::tuple<at::Tensor, at::Tensor, at::Tensor> fused_self_attention_bw(const at::Tensor &dout, const at::Tensor &q,
                                                                        const at::Tensor &k, const at::Tensor &v,
                                                                        const at::Tensor &out_m,
@@ -269,60 +339,43 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> fused_self_attention_bw(const at:
 
     TORCH_CHECK(q.is_cuda(), "fused_self_attention_bw: tensors must be on the CPU or a ROCm device, got ",
                 q.device());
-    const int32_t dt = to_pmkl_dtype(q.scalar_type());
-    TORCH_CHECK(pmkl_attn_bwd_supported(dt, D), "fused_self_attention_bw: the device backward supports float32, ",
-                "float16 and bfloat16 with head_dim 32, 64 or 128, got ", q.scalar_type(), " head_dim ", D);
-    // Gradients come back contiguous [B, H, S, D]; the kernels write every element.
-    auto gopts = q.options().memory_format(at::MemoryFormat::Contiguous);
-    auto dq = at::empty({B, H, S, D}, gopts);
-    auto dk = at::empty({B, H, S, D}, gopts);
-    auto dv = at::empty({B, H, S, D}, gopts);
-    if (B * H * S == 0) return std::forward_as_tuple(dq, dk, dv);
-    const int32_t mdt = to_pmkl_dtype(out_m.scalar_type());
-    TORCH_CHECK(out_m.scalar_type() == out_l.scalar_type() && (mdt == dt || mdt == PMKL_DTYPE_F32),
-                "fused_self_attention_bw: out_m / out_l must be in the tensors' dtype or float32");
+    return device_backward(dout, q, k, v, at::Tensor(), out_m, out_l, is_causal);
+}
 
-    c10::OptionalDeviceGuard guard(q.device());
-    auto mc = out_m.contiguous(), lc = out_l.contiguous();
-    // Strided views go to the kernels as they are; only a layout the kernels
-    // cannot address (head_dim not contiguous, strides or base not 16-byte
-    // aligned) is copied.
-    auto qd = device_view(q), kd = device_view(k), vd = device_view(v), dod = device_view(dout);
-    const uint64_t ws_bytes = pmkl_attn_bwd_workspace_size(B, H, S);
-    auto ws = at::empty({(int64_t)((ws_bytes + 3) / 4)}, q.options().dtype(at::kFloat));
-    pmkl_attn_bwd_args a;
-    std::memset(&a, 0, sizeof(a));
-    a.dout = dod.data_ptr();
-    a.q = qd.data_ptr();
-    a.k = kd.data_ptr();
-    a.v = vd.data_ptr();
-    fill_strides(a.dout_strides, dod);
-    fill_strides(a.q_strides, qd);
-    fill_strides(a.k_strides, kd);
-    fill_strides(a.v_strides, vd);
-    fill_strides(a.dq_strides, dq);
-    fill_strides(a.dk_strides, dk);
-    fill_strides(a.dv_strides, dv);
-    a.o = nullptr;
-    a.m = mc.data_ptr();
-    a.l = lc.data_ptr();
-    a.dq = dq.data_ptr();
-    a.dk = dk.data_ptr();
-    a.dv = dv.data_ptr();
-    a.workspace = ws.data_ptr();
-    a.workspace_bytes = (uint64_t)ws.numel() * 4;
-    a.dtype = dt;
-    a.ml_dtype = mdt;
-    a.batch = B;
-    a.heads = H;
-    a.seq_len = S;
-    a.head_dim = D;
-    a.scale = 0.f;
-    a.is_causal = is_causal ? 1 : 0;
-    hipStream_t stream = c10::hip::getCurrentHIPStream(q.device().index()).stream();
-    const int rc = pmkl_attn_bwd(&a, (void *)stream);
-    TORCH_CHECK(rc == PMKL_OK, "fused_self_attention_bw: ", pmkl_last_error());
-    return std::forward_as_tuple(dq, dk, dv);
+// The autograd entry on device tensors: what the Python autograd function of
+// pmkl_function does there (same outputs, same saved tensors, gradients of out
+// only), in native code.  A training step of a small problem is bound by the
+// host: the Python function, its argument binding and the backward's argument
+// block took ~140 us against ~40 us of kernels.  Gradients that nothing
+// produced are not materialised (two fill launches for out_m's and out_l's).
+class FusedSelfAttention : public torch::autograd::Function<FusedSelfAttention> {
+public:
+    static torch::autograd::variable_list forward(torch::autograd::AutogradContext *ctx, const at::Tensor &q,
+                                                  const at::Tensor &k, const at::Tensor &v, bool is_causal) {
+        at::Tensor out, out_m, out_l;
+        std::tie(out, out_m, out_l) = fused_self_attention_fw(q, k, v, is_causal);
+        ctx->save_for_backward({q, k, v, out, out_m, out_l});
+        ctx->saved_data["is_causal"] = is_causal;
+        ctx->set_materialize_grads(false);
+        return {out, out_m, out_l};
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx,
+                                                   torch::autograd::variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        const at::Tensor &q = saved[0], &out = saved[3];
+        // without a gradient of out its zeros, as the Python function sees them
+        const at::Tensor dout = grads[0].defined() ? grads[0] : at::zeros_like(out);
+        at::Tensor dq, dk, dv;
+        std::tie(dq, dk, dv) = device_backward(dout, q, saved[1], saved[2], out, saved[4], saved[5],
+                                               ctx->saved_data["is_causal"].toBool());
+        return {dq, dk, dv, at::Tensor()};
+    }
+};
+
+std::tuple<at::Tensor, at::Tensor, at::Tensor> fused_self_attention_autograd(const at::Tensor &q, const at::Tensor &k,
+                                                                             const at::Tensor &v, bool is_causal) {
+    auto r = FusedSelfAttention::apply(q, k, v, is_causal);
+    return std::make_tuple(r[0], r[1], r[2]);
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -331,4 +384,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("fused_self_attention_bw", &fused_self_attention_bw, "fused_self_attention_bw",
           pybind11::arg("dout"), pybind11::arg("q"), pybind11::arg("k"), pybind11::arg("v"),
           pybind11::arg("out_m"), pybind11::arg("out_l"), pybind11::arg("is_causal"));
+    m.def("fused_self_attention_autograd", &fused_self_attention_autograd,
+          "fused_self_attention_fw with the backward recorded (device tensors)", pybind11::arg("q"),
+          pybind11::arg("k"), pybind11::arg("v"), pybind11::arg("is_causal"));
 }

@@ -5,9 +5,9 @@ Same API as the reference pmkl_pytorch_ext/pmkl_function/__init__.py:1-33:
 ``(out, out_m, out_l)`` (the parameter really is spelled ``is_casual``).
 
 Dispatch:
-  * ROCm device tensors -> the gfx950 kernels (new: the reference raises
-    NotImplementedError for anything that is not a CPU tensor with debug=True,
-    __init__.py:15-18);
+  * ROCm device tensors -> the gfx950 kernels, recorded by the extension's
+    native autograd function (new: the reference raises NotImplementedError
+    for anything that is not a CPU tensor with debug=True, __init__.py:15-18);
   * CPU tensors with debug=True -> the operator's CPU body, as in the
     reference;
   * anything else -> NotImplementedError, as in the reference.
@@ -65,4 +65,11 @@ class fused_self_attention_(Function):
         return dq, dk, dv, None, None
 
 
-fused_self_attention = fused_self_attention_.apply
+def fused_self_attention(q, k, v, is_casual, debug=False):
+    # Device tensors take the same function in native code (a step of a small
+    # problem is bound by the host).  Where PyTorch looks into Python autograd
+    # functions (torch.func transforms, tracing, compilation) it gets that one.
+    if q.is_cuda and not (torch.compiler.is_compiling() or torch.jit.is_tracing()
+                          or torch._C._are_functorch_transforms_active()):
+        return pmkl_pytorch_ext.fused_self_attention_autograd(q, k, v, is_casual)
+    return fused_self_attention_.apply(q, k, v, is_casual, debug)
