@@ -26,8 +26,9 @@
 // so that a lane half owns 16 consecutive streamed rows, P and dS packed
 // straight into the B operand of the next product, and the LDS transpose read
 // ds_read_b64_tr_b16 for operands needed with the other orientation.  A
-// streamed tensor read both as rows and transposed is kept in LDS twice, once
-// per swizzle, so both reads are bank-conflict free.
+// streamed tile is kept in LDS once, with one swizzle (swz_b) under which both
+// reads are bank-conflict free; a copy per read cost B4 H32 S4096 D128 1,062 /
+// 1,338 us (dQ / dK/dV) against 1,033 / 1,268.
 #pragma once
 
 #include "attn_fwd_kernels.hpp"
@@ -60,16 +61,17 @@ __device__ __forceinline__ T *bwd_head(const BwdParams &p, const void *base, int
     return (T *)base + (int64_t)b * p.sb[t] + (int64_t)h * p.sh[t];
 }
 
-// Waves per workgroup: 8 (two per SIMD) where the registers of a wave fit in
-// 256, else 4 (one per SIMD, up to 512 registers): at head_dim 128 the
-// pipelined dQ loop (two score sets) and the dK/dV accumulators.
-template <int D> constexpr int bwd_waves_dq() { return D >= 128 ? 4 : 8; }
-template <int D> constexpr int bwd_waves_dkdv() { return D >= 128 ? 4 : 8; }
+// Waves per workgroup: one per SIMD, with up to 512 registers at head_dim 128
+// (the pipelined dQ loop's two score sets, the dK/dV accumulators), 256 below,
+// where two workgroups share a CU.  (One workgroup of eight waves instead runs
+// all their phases in step: B64 H8 S256 D32 19.4 / 22.0 us against 16.8 / 17.4.)
+template <int D> constexpr int bwd_waves_dq() { return 4; }
+template <int D> constexpr int bwd_waves_dkdv() { return 4; }
 
 // 16-byte chunk (logical chunk pc of row `row`) staging of a 64-row tile:
 // loads go to registers ahead of use (the dK/dV pass one tile ahead, the
 // dQ pass's plain loop below head_dim 128), LDS writes place the chunk at its
-// swizzled position in each layout the tensor is read with; the dQ pass at
+// swizzled position; the dQ pass at
 // head_dim 128 moves the chunks by LDS DMA instead.
 template <typename T, int D, int NW_>
 struct BwdTile {
@@ -92,7 +94,21 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t bwd_rows_rsrc(const T *base, i
                                              (int)((rows - 1) * ss + D) * (int)sizeof(T), 0x00020000);
 }
 
-// A-operand fragment (rows) of a 32-row block from a tile stored with swz_k:
+// XOR swizzle of the 16-byte chunks of a streamed tile's rows (CPR chunks per
+// row), one for both ways the tile is read.  Rows (ds_read_b128): 16 lanes read
+// one chunk of the rows r, r + 1 .. r + 3 and the same + 16, + 4, + 20, which
+// must lie in 16 different 16-byte slots of the 64 banks.  Transposed
+// (ds_read_b64_tr_b16): 32 lanes read four neighbouring chunks of the rows r ..
+// r + 3, again 16 different slots.  So the bits of r & 3 that a row's place in
+// the banks does not hold go above the chunk's low two bits, bits 4 and 2 below.
+template <int CPR> __device__ __forceinline__ int swz_b(int row) {
+    const int low = ((row >> 4) & 1) | (((row >> 2) & 1) << 1);
+    if constexpr (CPR >= 16) return low | ((row & 3) << 2);
+    if constexpr (CPR == 8) return low | (((row >> 1) & 1) << 2);
+    return low;
+}
+
+// A-operand fragment (rows) of a 32-row block from a tile stored with swz_b:
 // lane reads row 32 blk + key_of_arow(col), head_dim 16 dk + 8 hi .. +7.
 template <typename T, int D>
 __device__ __forceinline__ typename Elt16<T>::frag bwd_row_frag(const T *tile, int blk, int dk, int arow, int hi) {
@@ -100,11 +116,11 @@ __device__ __forceinline__ typename Elt16<T>::frag bwd_row_frag(const T *tile, i
     const int row = 32 * blk + arow;
     const int x = 2 * dk + hi;
     return __builtin_bit_cast(typename Elt16<T>::frag,
-                              *(const u32x4_t *)(tile + row * D + 8 * (x ^ swz_k<CPR>(row))));
+                              *(const u32x4_t *)(tile + row * D + 8 * (x ^ swz_b<CPR>(row))));
 }
 
 // A-operand fragment of the transpose (head_dim x 16 streamed rows) from a
-// tile stored with swz_v: 32 head-dim columns 32 db .., streamed rows of the
+// tile stored with swz_b: 32 head-dim columns 32 db .., streamed rows of the
 // 16-row block c of the 32-row block blk, in the order that matches a B
 // operand packed from registers 8c .. 8c+7 of the key_of_arow layout.
 template <typename T, int D>
@@ -116,8 +132,8 @@ __device__ __forceinline__ typename Elt16<T>::frag bwd_tr_frag(const T *tile, in
     const int r0 = 32 * blk + 8 * c + vrow0;
     const int cc = 32 * db + vcol0;
     const int ch = cc >> 3, part = cc & 7;
-    const T *a0 = tile + r0 * D + 8 * (ch ^ swz_v<CPR>(r0)) + part;
-    const T *a1 = tile + (r0 + 4) * D + 8 * (ch ^ swz_v<CPR>(r0 + 4)) + part;
+    const T *a0 = tile + r0 * D + 8 * (ch ^ swz_b<CPR>(r0)) + part;
+    const T *a1 = tile + (r0 + 4) * D + 8 * (ch ^ swz_b<CPR>(r0 + 4)) + part;
     s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)a0);
     s16x4_t hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)a1);
     return __builtin_bit_cast(typename Elt16<T>::frag,
@@ -143,7 +159,7 @@ __device__ __forceinline__ void bwd_lds_dma16(__amdgpu_buffer_rsrc_t r, int off,
 // pass 1: dQ (and the row vectors D_n, log2-sum-exp)
 // ---------------------------------------------------------------------------
 template <typename T, int D, bool CAUSAL>
-__global__ __launch_bounds__(bwd_waves_dq<D>() * 64, 1) void attn_bwd_dq_kernel(BwdParams p) {
+__global__ __launch_bounds__(bwd_waves_dq<D>() * 64, D >= 128 ? 1 : 2) void attn_bwd_dq_kernel(BwdParams p) {
     using E = Elt16<T>;
     using frag = typename E::frag;
     using TL = BwdTile<T, D, bwd_waves_dq<D>()>;
@@ -155,7 +171,7 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, 1) void attn_bwd_dq_kernel(
     // The software-pipelined loop (head_dim 128, one wave per SIMD) keeps three
     // tiles in LDS, the plain loop two.
     constexpr bool PIPE = D >= 128;
-    __shared__ __attribute__((aligned(16))) T smem[PIPE ? 3 : 2][3][BN * D];   // [stage][K swz_k, K swz_v, V swz_k]
+    __shared__ __attribute__((aligned(16))) T smem[PIPE ? 3 : 2][2][BN * D];   // [stage][K, V]
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -202,14 +218,13 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, 1) void attn_bwd_dq_kernel(
     // bytes layout_base + 16 THREADS j + 1024 wave + 16 lane) with the logical
     // chunk that the layout's XOR swizzle places there. ----
     constexpr int TILE_BYTES = BN * D * (int)sizeof(T);
-    int doffk[LOADS], doffkt[LOADS], doffv[LOADS];   // K rows, K transposed layout, V rows
+    int doffk[LOADS], doffv[LOADS];
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) {
         const int sl = j * kBwdThreads + tid;
         const int row = sl / CPR, pp = sl % CPR;
-        doffk[j] = (row * kss + 8 * (pp ^ swz_k<CPR>(row))) * (int)sizeof(T);
-        doffkt[j] = (row * kss + 8 * (pp ^ swz_v<CPR>(row))) * (int)sizeof(T);
-        doffv[j] = (row * vss + 8 * (pp ^ swz_k<CPR>(row))) * (int)sizeof(T);
+        doffk[j] = (row * kss + 8 * (pp ^ swz_b<CPR>(row))) * (int)sizeof(T);
+        doffv[j] = (row * vss + 8 * (pp ^ swz_b<CPR>(row))) * (int)sizeof(T);
     }
     const unsigned lds_w = (unsigned)(uintptr_t)(__attribute__((address_space(3))) T *)&smem[0][0][0] + 1024u * wave;
     // All DMAs of tile kt into stage kt % 3 (rows past S read as zero).
@@ -217,12 +232,11 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, 1) void attn_bwd_dq_kernel(
         static_assert(!PIPE || !PARTIAL, "the DMA staging covers whole tiles");
         const auto kr = bwd_rows_rsrc<T, D>(kg, kt * BN, S, kss);
         const auto vr = bwd_rows_rsrc<T, D>(vg, kt * BN, S, vss);
-        const unsigned base = lds_w + (unsigned)((kt % 3) * 3 * TILE_BYTES);
+        const unsigned base = lds_w + (unsigned)((kt % 3) * 2 * TILE_BYTES);
         bwd_static_for<0, LOADS>([&](auto j_c) __attribute__((always_inline)) {
             constexpr int J = decltype(j_c)::value;
             bwd_lds_dma16<0 * TILE_BYTES + 16 * kBwdThreads * J>(kr, doffk[J], base);
-            bwd_lds_dma16<1 * TILE_BYTES + 16 * kBwdThreads * J>(kr, doffkt[J], base);
-            bwd_lds_dma16<2 * TILE_BYTES + 16 * kBwdThreads * J>(vr, doffv[J], base);
+            bwd_lds_dma16<1 * TILE_BYTES + 16 * kBwdThreads * J>(vr, doffv[J], base);
         });
     };
     // The DMAs are inline asm: their completion is waited for explicitly,
@@ -259,9 +273,8 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, 1) void attn_bwd_dq_kernel(
             const int sl = j * kBwdThreads + tid;
             if (!PARTIAL || sl < TL::CHUNKS) {
                 const int row = sl / CPR, pc = sl % CPR;
-                *(u32x4_t *)(&smem[st][0][row * D + 8 * (pc ^ swz_k<CPR>(row))]) = kreg2[SET][j];
-                *(u32x4_t *)(&smem[st][1][row * D + 8 * (pc ^ swz_v<CPR>(row))]) = kreg2[SET][j];
-                *(u32x4_t *)(&smem[st][2][row * D + 8 * (pc ^ swz_k<CPR>(row))]) = vreg2[SET][j];
+                *(u32x4_t *)(&smem[st][0][row * D + 8 * (pc ^ swz_b<CPR>(row))]) = kreg2[SET][j];
+                *(u32x4_t *)(&smem[st][1][row * D + 8 * (pc ^ swz_b<CPR>(row))]) = vreg2[SET][j];
             }
         }
     };
@@ -284,7 +297,7 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, 1) void attn_bwd_dq_kernel(
     constexpr int NSD = 4 * NDK;
     auto sd_frag = [&](int st, int m) __attribute__((always_inline)) {
         const int dk = m >> 2, kb = (m >> 1) & 1, which = m & 1;
-        return bwd_row_frag<T, D>(smem[st][which ? 2 : 0], kb, dk, arow, hi);
+        return bwd_row_frag<T, D>(smem[st][which], kb, dk, arow, hi);
     };
     auto sd_mma = [&](f32x16_t (&sv)[2], f32x16_t (&dpv)[2], int m, frag a) __attribute__((always_inline)) {
         const int dk = m >> 2, kb = (m >> 1) & 1, which = m & 1;
@@ -338,7 +351,7 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, 1) void attn_bwd_dq_kernel(
                 // One stream of fragments through the ring: the S^T, dP^T
                 // row fragments of tile kt+1, then (dQ pass) the transposed K
                 // fragments of tile kt, so the first dQ MFMAs find theirs read.
-                const T *Kv = smem[st][1];
+                const T *Kv = smem[st][0];
                 constexpr int NQ = PASS == 1 ? 4 * NDB : 0;
                 static_assert(NSD % RING == 0, "the dQ MFMAs continue the ring");
                 // dQ MFMA m is (kb, cc, db) = (m / (2 NDB), (m / NDB) % 2, m % NDB)
@@ -423,9 +436,8 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, 1) void attn_bwd_dq_kernel(
             const bool need_mask = (CAUSAL && kbase + BN - 1 > q0w) || (kbase + BN > S);
             auto work = [&](auto mask_c) __attribute__((always_inline)) {
                 constexpr bool MASK = decltype(mask_c)::value;
-                const T *Kk = smem[SET][0];
-                const T *Kv = smem[SET][1];
-                const T *Vk = smem[SET][2];
+                const T *Kt = smem[SET][0];
+                const T *Vt = smem[SET][1];
                 f32x16_t s[2], dp[2];
 #pragma unroll
                 for (int kb = 0; kb < 2; ++kb) {
@@ -433,8 +445,8 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, 1) void attn_bwd_dq_kernel(
                     for (int r = 0; r < 16; ++r) s[kb][r] = dp[kb][r] = 0.f;
 #pragma unroll
                     for (int dk = 0; dk < NDK; ++dk) {
-                        s[kb] = E::mma(bwd_row_frag<T, D>(Kk, kb, dk, arow, hi), qf[dk], s[kb]);
-                        dp[kb] = E::mma(bwd_row_frag<T, D>(Vk, kb, dk, arow, hi), df[dk], dp[kb]);
+                        s[kb] = E::mma(bwd_row_frag<T, D>(Kt, kb, dk, arow, hi), qf[dk], s[kb]);
+                        dp[kb] = E::mma(bwd_row_frag<T, D>(Vt, kb, dk, arow, hi), df[dk], dp[kb]);
                     }
                 }
                 // register r of block kb holds key kbase + 32 kb + 16 hi + r
@@ -468,7 +480,7 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, 1) void attn_bwd_dq_kernel(
                             const frag bfr = __builtin_bit_cast(frag, bw);
 #pragma unroll
                             for (int db = 0; db < NDB; ++db)
-                                acc[db] = E::mma(bwd_tr_frag<T, D>(Kv, kb, cc, db, vrow0, vcol0), bfr, acc[db]);
+                                acc[db] = E::mma(bwd_tr_frag<T, D>(Kt, kb, cc, db, vrow0, vcol0), bfr, acc[db]);
                         }
                 }
             };
@@ -547,7 +559,7 @@ __device__ __forceinline__ int bwd_dkdv_mlim(int qbase, int k0w, int kj, int hi)
 }
 
 template <typename T, int D, bool CAUSAL>
-__global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, 1) void attn_bwd_dkdv_kernel(BwdParams p) {
+__global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, D >= 128 ? 1 : 2) void attn_bwd_dkdv_kernel(BwdParams p) {
     using E = Elt16<T>;
     using frag = typename E::frag;
     using TL = BwdTile<T, D, bwd_waves_dkdv<D>()>;
@@ -556,8 +568,8 @@ __global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, 1) void attn_bwd_dkdv_ker
     constexpr bool PARTIAL = TL::PARTIAL;
     constexpr int NDB = D / 32, NDK = D / 16;
 
-    // [stage][Q swz_k, Q swz_v, dout swz_k, dout swz_v]; row vectors [stage][lse2, D_n]
-    __shared__ __attribute__((aligned(16))) T smem[2][4][BN * D];
+    // [stage][Q, dout]; row vectors [stage][lse2, D_n]
+    __shared__ __attribute__((aligned(16))) T smem[2][2][BN * D];
     __shared__ __attribute__((aligned(16))) float svec[2][2][BN];
 
     const int tid = threadIdx.x;
@@ -629,10 +641,8 @@ __global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, 1) void attn_bwd_dkdv_ker
             const int sl = j * kBwdThreads + tid;
             if (!PARTIAL || sl < TL::CHUNKS) {
                 const int row = sl / CPR, pc = sl % CPR;
-                *(u32x4_t *)(&smem[st][0][row * D + 8 * (pc ^ swz_k<CPR>(row))]) = qreg[j];
-                *(u32x4_t *)(&smem[st][1][row * D + 8 * (pc ^ swz_v<CPR>(row))]) = qreg[j];
-                *(u32x4_t *)(&smem[st][2][row * D + 8 * (pc ^ swz_k<CPR>(row))]) = oreg[j];
-                *(u32x4_t *)(&smem[st][3][row * D + 8 * (pc ^ swz_v<CPR>(row))]) = oreg[j];
+                *(u32x4_t *)(&smem[st][0][row * D + 8 * (pc ^ swz_b<CPR>(row))]) = qreg[j];
+                *(u32x4_t *)(&smem[st][1][row * D + 8 * (pc ^ swz_b<CPR>(row))]) = oreg[j];
             }
         }
         if (tid < 2 * BN) svec[st][tid >> 6][tid & (BN - 1)] = vreg;
@@ -669,10 +679,8 @@ __global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, 1) void attn_bwd_dkdv_ker
         // causal: the tile holds a query at or past the wave's first key
         const bool wave_needed = wave_active && (!CAUSAL || qbase + BN - 1 >= k0w);
         if (wave_needed) {
-            const T *Qk = smem[SET][0];
-            const T *Qv = smem[SET][1];
-            const T *Ok = smem[SET][2];
-            const T *Ov = smem[SET][3];
+            const T *Qt = smem[SET][0];
+            const T *Ot = smem[SET][1];
             const float *lse2s = svec[SET][0];
             const float *drows = svec[SET][1];
             if constexpr (D >= 128) {
@@ -690,10 +698,10 @@ __global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, 1) void attn_bwd_dkdv_ker
                 auto frag_at = [&](int n) __attribute__((always_inline)) {
                     if (n < 2 * NSQ) {
                         const int qb = n / NSQ, j = n % NSQ;
-                        return bwd_row_frag<T, D>((j & 1) ? Ok : Qk, qb, j >> 1, arow, hi);
+                        return bwd_row_frag<T, D>((j & 1) ? Ot : Qt, qb, j >> 1, arow, hi);
                     }
                     const int m = n - 2 * NSQ, qb = m / NGQ, j = m % NGQ;
-                    return bwd_tr_frag<T, D>((j & 1) ? Qv : Ov, qb, j / (2 * NDB), (j >> 1) % NDB, vrow0, vcol0);
+                    return bwd_tr_frag<T, D>((j & 1) ? Qt : Ot, qb, j / (2 * NDB), (j >> 1) % NDB, vrow0, vcol0);
                 };
                 // register r of block qb holds query qbase + 32 qb + 16 hi + r;
                 // the causal mask keeps it iff 32 qb + r >= mlim (bwd_dkdv_mlim)
@@ -768,7 +776,7 @@ __global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, 1) void attn_bwd_dkdv_ker
                 // RING MFMAs ahead
                 constexpr int RING = 2, NSD = 4 * NDK;
                 auto sd_frag = [&](int m) __attribute__((always_inline)) {
-                    return bwd_row_frag<T, D>((m & 1) ? Ok : Qk, (m >> 1) & 1, m >> 2, arow, hi);
+                    return bwd_row_frag<T, D>((m & 1) ? Ot : Qt, (m >> 1) & 1, m >> 2, arow, hi);
                 };
                 f32x16_t s[2], dp[2];
                 {
@@ -815,7 +823,7 @@ __global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, 1) void attn_bwd_dkdv_ker
                 constexpr int NGR = 8 * NDB;
                 auto gr_frag = [&](int m) __attribute__((always_inline)) {
                     const int db = (m >> 1) % NDB, cc = (m / (2 * NDB)) & 1, qb = m / (4 * NDB);
-                    return bwd_tr_frag<T, D>((m & 1) ? Qv : Ov, qb, cc, db, vrow0, vcol0);
+                    return bwd_tr_frag<T, D>((m & 1) ? Qt : Ot, qb, cc, db, vrow0, vcol0);
                 };
                 {
                     frag ring[RING];
