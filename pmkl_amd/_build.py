@@ -44,7 +44,8 @@ def _run(cmd: list[str], cwd: Path = ROOT) -> None:
 
 
 CAPI_SOURCES = ("attn_capi.hip", "softmax_capi.hip", "attn_fwd_w64_bf16_causal.hip", "attn_fwd_w64_bf16_full.hip",
-                "attn_fwd_w64_f16_causal.hip", "attn_fwd_w64_f16_full.hip")
+                "attn_fwd_w64_f16_causal.hip", "attn_fwd_w64_f16_full.hip", "attn_bwd_split_bf16.hip",
+                "attn_bwd_split_f16.hip")
 
 
 def build_capi() -> Path:

@@ -12,7 +12,7 @@
 // which is the reference's per-(n, j) sum (:101-124) regrouped.
 //
 // Two passes, neither with atomics:
-//   attn_bwd_dq_kernel    a workgroup owns 32 query rows per wave;
+//   attn_bwd_dq_kernel    a workgroup owns 32 query rows per wave (KS = 1);
 //                         K and V tiles of 64 keys stream through LDS.  One
 //                         loop over the keys gives D_n (skipped when the
 //                         caller passes O: D_n = dout_n . o_n), a second one
@@ -21,6 +21,12 @@
 //   attn_bwd_dkdv_kernel  a workgroup owns 32 key rows per wave; Q, dO tiles of 64
 //                         queries and their two row vectors stream through
 //                         LDS; dK, dV accumulate in registers.
+// KS = 2 (chosen where workgroups are few): a workgroup owns 64 rows and two
+// waves share 32 of them, each with half of the streamed rows (dQ: a 32-key
+// block of every tile; dK/dV: 64 of a tile's 128 queries), so the chain of
+// dependent tiles, which sets the time of a small grid, is half as long and
+// twice as many CUs work; the waves' sums meet in LDS.  B2 H8 S2047 D128 causal
+// without O, whole call 158 -> 131 us, B1 H2 S4096 D128 288 -> 192.
 // Both use the forward's layouts (attn_fwd_kernels.hpp): transposed products
 // with the owned rows as the MFMA column, the A-row permutation key_of_arow
 // so that a lane half owns 16 consecutive streamed rows, P and dS packed
@@ -61,7 +67,7 @@ __device__ __forceinline__ T *bwd_head(const BwdParams &p, const void *base, int
     return (T *)base + (int64_t)b * p.sb[t] + (int64_t)h * p.sh[t];
 }
 
-// Waves per workgroup: one per SIMD, with up to 512 registers at head_dim 128
+// Waves per workgroup (32 / KS owned rows each): one per SIMD, with up to 512 registers at head_dim 128
 // (the pipelined dQ loop's two score sets, the dK/dV accumulators), 256 below,
 // where two workgroups share a CU.  (One workgroup of eight waves instead runs
 // all their phases in step: B64 H8 S256 D32 19.4 / 22.0 us against 16.8 / 17.4.)
@@ -73,12 +79,12 @@ template <int D> constexpr int bwd_waves_dkdv() { return 4; }
 // dQ pass's plain loop below head_dim 128), LDS writes place the chunk at its
 // swizzled position; the dQ pass at
 // head_dim 128 moves the chunks by LDS DMA instead.
-template <typename T, int D, int NW_>
+template <typename T, int D, int NW_, int KS = 1, int BN_ = 64>
 struct BwdTile {
     static constexpr int NW = NW_;
     static constexpr int THREADS = NW * 64;
-    static constexpr int ROWS = 32 * NW;        // owned rows per workgroup
-    static constexpr int BN = 64;
+    static constexpr int ROWS = 32 * NW / KS;   // owned rows per workgroup
+    static constexpr int BN = BN_;              // streamed rows per tile
     static constexpr int CPR = D / 8;
     static constexpr int CHUNKS = BN * CPR;
     static constexpr int LOADS = (CHUNKS + THREADS - 1) / THREADS;
@@ -87,9 +93,9 @@ struct BwdTile {
 
 // Buffer resource of the rows [r0, S) of a [S, D] matrix with row stride ss
 // elements: rows past S read as zero.
-template <typename T, int D>
+template <typename T, int D, int ROWS = 64>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t bwd_rows_rsrc(const T *base, int r0, int S, int ss) {
-    const int rows = min(64, S - r0);
+    const int rows = min(ROWS, S - r0);
     return __builtin_amdgcn_make_buffer_rsrc((void *)(base + (int64_t)r0 * ss), (short)0,
                                              (int)((rows - 1) * ss + D) * (int)sizeof(T), 0x00020000);
 }
@@ -158,20 +164,22 @@ __device__ __forceinline__ void bwd_lds_dma16(__amdgpu_buffer_rsrc_t r, int off,
 // ---------------------------------------------------------------------------
 // pass 1: dQ (and the row vectors D_n, log2-sum-exp)
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool CAUSAL>
+template <typename T, int D, bool CAUSAL, int KS = 1>
 __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, D >= 128 ? 1 : 2) void attn_bwd_dq_kernel(BwdParams p) {
     using E = Elt16<T>;
     using frag = typename E::frag;
-    using TL = BwdTile<T, D, bwd_waves_dq<D>()>;
+    using TL = BwdTile<T, D, bwd_waves_dq<D>(), KS>;
     constexpr int BN = TL::BN, CPR = TL::CPR, LOADS = TL::LOADS;
     constexpr int kBwdThreads = TL::THREADS, kBwdRows = TL::ROWS;
     constexpr bool PARTIAL = TL::PARTIAL;
     constexpr int NDB = D / 32, NDK = D / 16;
+    constexpr int NKB = 2 / KS;   // 32-key blocks of a tile per wave
 
     // The software-pipelined loop (head_dim 128, one wave per SIMD) keeps three
     // tiles in LDS, the plain loop two.
     constexpr bool PIPE = D >= 128;
     __shared__ __attribute__((aligned(16))) T smem[PIPE ? 3 : 2][2][BN * D];   // [stage][K, V]
+    __shared__ float dpart[KS > 1 ? TL::NW : 1][32];   // split: each wave's part of D_n
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -191,7 +199,8 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, D >= 128 ? 1 : 2) void attn
     const int qss = p.ss[BQ], kss = p.ss[BK], vss = p.ss[BV], doss = p.ss[BDOUT];
 
     const int q0 = qt * kBwdRows;
-    const int q0w = q0 + 32 * wave;
+    const int q0w = q0 + 32 * (wave / KS);
+    const int kb0 = KS > 1 ? wave % KS : 0;   // this wave's first block of a tile
     const int qi = q0w + col;                 // this lane's query row
     const int qrow = min(qi, S - 1);
     const int last_key = CAUSAL ? min(q0 + kBwdRows - 1, S - 1) : S - 1;
@@ -293,19 +302,19 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, D >= 128 ? 1 : 2) void attn
         for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
 
     // Scores S^T and dP^T of a tile: MFMA m (0 .. NSD-1) is (dk, kb, which)
-    // = (m / 4, (m / 2) % 2, m % 2), i.e. four interleaved accumulator chains.
-    constexpr int NSD = 4 * NDK;
+    // = (m / (2 NKB), (m / 2) % NKB, m % 2), i.e. 2 NKB interleaved accumulator chains.
+    constexpr int NSD = 2 * NKB * NDK;
     auto sd_frag = [&](int st, int m) __attribute__((always_inline)) {
-        const int dk = m >> 2, kb = (m >> 1) & 1, which = m & 1;
-        return bwd_row_frag<T, D>(smem[st][which], kb, dk, arow, hi);
+        const int dk = m / (2 * NKB), kb = (m >> 1) % NKB, which = m & 1;
+        return bwd_row_frag<T, D>(smem[st][which], kb0 + kb, dk, arow, hi);
     };
-    auto sd_mma = [&](f32x16_t (&sv)[2], f32x16_t (&dpv)[2], int m, frag a) __attribute__((always_inline)) {
-        const int dk = m >> 2, kb = (m >> 1) & 1, which = m & 1;
+    auto sd_mma = [&](f32x16_t (&sv)[NKB], f32x16_t (&dpv)[NKB], int m, frag a) __attribute__((always_inline)) {
+        const int dk = m / (2 * NKB), kb = (m >> 1) % NKB, which = m & 1;
         if (which) dpv[kb] = E::mma(a, df[dk], dk == 0 ? f32x16_t{} : dpv[kb]);
         else sv[kb] = E::mma(a, qf[dk], dk == 0 ? f32x16_t{} : sv[kb]);
     };
     // All scores of tile (stage st), fragments read one MFMA ahead.
-    auto sd_tile = [&](f32x16_t (&sv)[2], f32x16_t (&dpv)[2], int st) __attribute__((always_inline)) {
+    auto sd_tile = [&](f32x16_t (&sv)[NKB], f32x16_t (&dpv)[NKB], int st) __attribute__((always_inline)) {
         frag a = sd_frag(st, 0);
 #pragma unroll
         for (int m = 0; m < NSD; ++m) {
@@ -322,23 +331,23 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, D >= 128 ? 1 : 2) void attn
     // fragments read RING MFMAs ahead through one ring.  One barrier per
     // tile, after the wait for the DMAs.
     constexpr int RING = 4;
-    constexpr int NUNIT = 16;   // softmax units of a tile: (kb, register pair)
+    constexpr int NUNIT = 8 * NKB;   // softmax units of a tile: (kb, register pair)
     auto key_loop = [&](auto pass_c) __attribute__((always_inline)) {
         constexpr int PASS = decltype(pass_c)::value;
         dma_tile(0);
         if (nt > 1) dma_tile(1);
         dma_wait_sync();
-        f32x16_t s0[2], dp0[2], s1[2], dp1[2];
+        f32x16_t s0[NKB], dp0[NKB], s1[NKB], dp1[NKB];
         if (wave_active) sd_tile(s0, dp0, 0);
 
-        auto step = [&](int kt, f32x16_t (&sc)[2], f32x16_t (&dpc)[2], f32x16_t (&sn)[2], f32x16_t (&dpn)[2])
+        auto step = [&](int kt, f32x16_t (&sc)[NKB], f32x16_t (&dpc)[NKB], f32x16_t (&sn)[NKB], f32x16_t (&dpn)[NKB])
                         __attribute__((always_inline)) {
             const int st = kt % 3, st1 = (kt + 1) % 3;
             // tile kt+2 into the stage of tile kt-1, which every wave finished
             // reading before the last barrier
             if (kt + 2 < nt) dma_tile(kt + 2);
             const int kbase = kt * BN;
-            const bool wave_needed = wave_active && (!CAUSAL || kbase <= q0w + 31);
+            const bool wave_needed = wave_active && (!CAUSAL || kbase + 32 * kb0 <= q0w + 31);
             // Two copies of the tile's work, with and without the mask (a
             // wave masks only its last tile, and the one past S): written
             // per score, the mask's compare and select cost ~130 scalar and
@@ -347,16 +356,16 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, D >= 128 ? 1 : 2) void attn
             auto work = [&](auto mask_c) __attribute__((always_inline)) {
                 constexpr bool MASK = decltype(mask_c)::value;
                 const int lim = CAUSAL ? min(qi, S - 1) : S - 1;
-                uint32_t dsk[2][8];
+                uint32_t dsk[NKB][8];
                 // One stream of fragments through the ring: the S^T, dP^T
                 // row fragments of tile kt+1, then (dQ pass) the transposed K
                 // fragments of tile kt, so the first dQ MFMAs find theirs read.
                 const T *Kv = smem[st][0];
-                constexpr int NQ = PASS == 1 ? 4 * NDB : 0;
+                constexpr int NQ = PASS == 1 ? 2 * NKB * NDB : 0;
                 static_assert(NSD % RING == 0, "the dQ MFMAs continue the ring");
                 // dQ MFMA m is (kb, cc, db) = (m / (2 NDB), (m / NDB) % 2, m % NDB)
                 auto kt_frag = [&](int m) __attribute__((always_inline)) {
-                    return bwd_tr_frag<T, D>(Kv, m / (2 * NDB), (m / NDB) & 1, m % NDB, vrow0, vcol0);
+                    return bwd_tr_frag<T, D>(Kv, kb0 + m / (2 * NDB), (m / NDB) & 1, m % NDB, vrow0, vcol0);
                 };
                 auto next_frag = [&](int n) __attribute__((always_inline)) {
                     return n < NSD ? sd_frag(st1, n) : kt_frag(n - NSD);
@@ -380,7 +389,7 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, D >= 128 ? 1 : 2) void attn
                     if ((m & 1) == 0) {
 #pragma unroll
                         for (int e = 0; e < 2; ++e) {
-                            const int key = kbase + 32 * kb + 16 * hi + r + e;
+                            const int key = kbase + 32 * (kb0 + kb) + 16 * hi + r + e;
                             const float sv = MASK && key > lim ? -INFINITY : sc[kb][r + e];
                             pv[e] = fast_exp2(__builtin_fmaf(sv, c, -lse2));
                         }
@@ -393,7 +402,7 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, D >= 128 ? 1 : 2) void attn
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 if (PASS == 1) {
-                    // dQ^T += K^T dS^T over the 4 blocks of 16 keys, the
+                    // dQ^T += K^T dS^T over the wave's blocks of 16 keys, the
                     // transposed K fragments continuing the ring
 #pragma unroll
                     for (int m = 0; m < NQ; ++m) {
@@ -431,35 +440,35 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, D >= 128 ? 1 : 2) void attn
             constexpr int SET = decltype(set_c)::value;
             gload2(min(kt + 2, nt - 1), set_c);
             const int kbase = kt * BN;
-            const bool wave_needed = wave_active && (!CAUSAL || kbase <= q0w + 31);
+            const bool wave_needed = wave_active && (!CAUSAL || kbase + 32 * kb0 <= q0w + 31);
             // masked and unmasked copies, as in the pipelined loop
             const bool need_mask = (CAUSAL && kbase + BN - 1 > q0w) || (kbase + BN > S);
             auto work = [&](auto mask_c) __attribute__((always_inline)) {
                 constexpr bool MASK = decltype(mask_c)::value;
                 const T *Kt = smem[SET][0];
                 const T *Vt = smem[SET][1];
-                f32x16_t s[2], dp[2];
+                f32x16_t s[NKB], dp[NKB];
 #pragma unroll
-                for (int kb = 0; kb < 2; ++kb) {
+                for (int kb = 0; kb < NKB; ++kb) {
 #pragma unroll
                     for (int r = 0; r < 16; ++r) s[kb][r] = dp[kb][r] = 0.f;
 #pragma unroll
                     for (int dk = 0; dk < NDK; ++dk) {
-                        s[kb] = E::mma(bwd_row_frag<T, D>(Kt, kb, dk, arow, hi), qf[dk], s[kb]);
-                        dp[kb] = E::mma(bwd_row_frag<T, D>(Vt, kb, dk, arow, hi), df[dk], dp[kb]);
+                        s[kb] = E::mma(bwd_row_frag<T, D>(Kt, kb0 + kb, dk, arow, hi), qf[dk], s[kb]);
+                        dp[kb] = E::mma(bwd_row_frag<T, D>(Vt, kb0 + kb, dk, arow, hi), df[dk], dp[kb]);
                     }
                 }
-                // register r of block kb holds key kbase + 32 kb + 16 hi + r
+                // register r of block kb holds key kbase + 32 (kb0 + kb) + 16 hi + r
                 const int lim = CAUSAL ? min(qi, S - 1) : S - 1;
-                uint32_t dsk[2][8];
+                uint32_t dsk[NKB][8];
 #pragma unroll
-                for (int kb = 0; kb < 2; ++kb)
+                for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
                     for (int r = 0; r < 16; r += 2) {
                         float pv[2];
 #pragma unroll
                         for (int e = 0; e < 2; ++e) {
-                            const int key = kbase + 32 * kb + 16 * hi + r + e;
+                            const int key = kbase + 32 * (kb0 + kb) + 16 * hi + r + e;
                             const float sv = MASK && key > lim ? -INFINITY : s[kb][r + e];
                             pv[e] = fast_exp2(__builtin_fmaf(sv, c, -lse2));
                         }
@@ -471,16 +480,16 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, D >= 128 ? 1 : 2) void attn
                         }
                     }
                 if (PASS == 1) {
-                    // dQ^T += K^T dS^T over the 4 blocks of 16 keys
+                    // dQ^T += K^T dS^T over the wave's blocks of 16 keys
 #pragma unroll
-                    for (int kb = 0; kb < 2; ++kb)
+                    for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
                         for (int cc = 0; cc < 2; ++cc) {
                             u32x4_t bw = {dsk[kb][4 * cc], dsk[kb][4 * cc + 1], dsk[kb][4 * cc + 2], dsk[kb][4 * cc + 3]};
                             const frag bfr = __builtin_bit_cast(frag, bw);
 #pragma unroll
                             for (int db = 0; db < NDB; ++db)
-                                acc[db] = E::mma(bwd_tr_frag<T, D>(Kt, kb, cc, db, vrow0, vcol0), bfr, acc[db]);
+                                acc[db] = E::mma(bwd_tr_frag<T, D>(Kt, kb0 + kb, cc, db, vrow0, vcol0), bfr, acc[db]);
                         }
                 }
             };
@@ -512,16 +521,34 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, D >= 128 ? 1 : 2) void attn
         if constexpr (PIPE) key_loop(std::integral_constant<int, 0>{});
         else key_loop_plain(std::integral_constant<int, 0>{});
         drow = half_sum(drow_part);
+        if constexpr (KS > 1) {   // the two waves' parts, added in one order
+            if (hi == 0) dpart[wave][col] = drow;
+            __syncthreads();
+            drow = dpart[wave & ~1][col] + dpart[wave | 1][col];
+        }
     }
-    if (hi == 0 && qi < S) {
+    if (hi == 0 && kb0 == 0 && qi < S) {
         p.lse2[(int64_t)bh * S + qi] = lse2;
         p.drow[(int64_t)bh * S + qi] = drow;
     }
     if constexpr (PIPE) key_loop(std::integral_constant<int, 1>{});
     else key_loop_plain(std::integral_constant<int, 1>{});
 
+    if constexpr (KS > 1) {
+        // the second wave's dQ^T through the tiles' LDS (every wave is past its
+        // last read of them), [row group][register][lane]
+        float *part = (float *)&smem[0][0][0] + (wave / KS) * (NDB * 1024) + lane;
+        if (kb0 == 1)
+#pragma unroll
+            for (int i = 0; i < NDB * 16; ++i) part[64 * i] = acc[i >> 4][i & 15];
+        __syncthreads();
+        if (kb0 == 0)
+#pragma unroll
+            for (int i = 0; i < NDB * 16; ++i) acc[i >> 4][i & 15] += part[64 * i];
+    }
+
     // ---- epilogue: dq = scale * dQ^T, lane = query column ----
-    if (wave_active && qi < S) {
+    if (wave_active && kb0 == 0 && qi < S) {
         T *row = dqg + (int64_t)qi * p.ss[BDQ];
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
@@ -558,11 +585,11 @@ __device__ __forceinline__ int bwd_dkdv_mlim(int qbase, int k0w, int kj, int hi)
     return CAUSAL && qbase < k0w + 31 ? kj - qbase - 16 * hi : -64;
 }
 
-template <typename T, int D, bool CAUSAL>
+template <typename T, int D, bool CAUSAL, int KS = 1>
 __global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, D >= 128 ? 1 : 2) void attn_bwd_dkdv_kernel(BwdParams p) {
     using E = Elt16<T>;
     using frag = typename E::frag;
-    using TL = BwdTile<T, D, bwd_waves_dkdv<D>()>;
+    using TL = BwdTile<T, D, bwd_waves_dkdv<D>(), KS, 64 * KS>;
     constexpr int BN = TL::BN, CPR = TL::CPR, LOADS = TL::LOADS;
     constexpr int kBwdThreads = TL::THREADS, kBwdRows = TL::ROWS;
     constexpr bool PARTIAL = TL::PARTIAL;
@@ -593,7 +620,8 @@ __global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, D >= 128 ? 1 : 2) void at
     const int qss = p.ss[BQ], doss = p.ss[BDOUT];
 
     const int k0 = ktile * kBwdRows;
-    const int k0w = k0 + 32 * wave;
+    const int k0w = k0 + 32 * (wave / KS);
+    const int qh = KS > 1 ? wave % KS : 0;    // this wave's 64 queries of a tile
     const int kj = k0w + col;                 // this lane's key row
     const int krow = min(kj, S - 1);
     const bool wave_active = k0w < S;
@@ -621,8 +649,8 @@ __global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, D >= 128 ? 1 : 2) void at
         goffo[j] = ((sl / CPR) * doss + 8 * (sl % CPR)) * (int)sizeof(T);
     }
     auto gload = [&](int qtl) __attribute__((always_inline)) {
-        const auto qr = bwd_rows_rsrc<T, D>(qg, qtl * BN, S, qss);
-        const auto orr = bwd_rows_rsrc<T, D>(dog, qtl * BN, S, doss);
+        const auto qr = bwd_rows_rsrc<T, D, BN>(qg, qtl * BN, S, qss);
+        const auto orr = bwd_rows_rsrc<T, D, BN>(dog, qtl * BN, S, doss);
 #pragma unroll
         for (int j = 0; j < LOADS; ++j)
             if (!PARTIAL || j * kBwdThreads + tid < TL::CHUNKS) {
@@ -645,7 +673,7 @@ __global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, D >= 128 ? 1 : 2) void at
                 *(u32x4_t *)(&smem[st][1][row * D + 8 * (pc ^ swz_b<CPR>(row))]) = oreg[j];
             }
         }
-        if (tid < 2 * BN) svec[st][tid >> 6][tid & (BN - 1)] = vreg;
+        if (tid < 2 * BN) svec[st][tid / BN][tid & (BN - 1)] = vreg;
     };
 
     const int arow = key_of_arow(col);
@@ -675,14 +703,14 @@ __global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, D >= 128 ? 1 : 2) void at
         // loaded into the same registers: one register set, a tile of latency.
         if (it + 1 < ntl) swrite(SET ^ 1);
         gload(min(qtl + 2, nq - 1));
-        const int qbase = qtl * BN;
-        // causal: the tile holds a query at or past the wave's first key
-        const bool wave_needed = wave_active && (!CAUSAL || qbase + BN - 1 >= k0w);
+        const int qbase = qtl * BN + 64 * qh;
+        // causal: the wave's 64 queries reach its first key
+        const bool wave_needed = wave_active && (!CAUSAL || qbase + 63 >= k0w) && (KS == 1 || qbase < S);
         if (wave_needed) {
-            const T *Qt = smem[SET][0];
-            const T *Ot = smem[SET][1];
-            const float *lse2s = svec[SET][0];
-            const float *drows = svec[SET][1];
+            const T *Qt = smem[SET][0] + 64 * D * qh;
+            const T *Ot = smem[SET][1] + 64 * D * qh;
+            const float *lse2s = svec[SET][0] + 64 * qh;
+            const float *drows = svec[SET][1] + 64 * qh;
             if constexpr (D >= 128) {
                 // Half-tile pipeline over the two 32-query blocks qb: one stream of
                 // NMM MFMAs in four phases,
@@ -849,6 +877,33 @@ __global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, D >= 128 ? 1 : 2) void at
     for (int it = 0; it < ntl; it += 2) {
         tile_step(std::integral_constant<int, 0>{}, it);
         if (it + 1 < ntl) tile_step(std::integral_constant<int, 1>{}, it + 1);
+    }
+
+    if constexpr (KS > 1) {
+        // The two waves' sums through the tiles' LDS (every wave is past its
+        // last read of them), [wave][register][lane]: the first wave hands over
+        // its dV^T and finishes dK, the second the other way round.
+        float *part = (float *)&smem[0][0][0] + lane;
+#pragma unroll
+        for (int i = 0; i < NDB * 16; ++i)
+            part[64 * i + wave * (NDB * 1024)] = qh ? dk_acc[i >> 4][i & 15] : dv_acc[i >> 4][i & 15];
+        __syncthreads();
+        if (!wave_active || kj >= S) return;
+        T *row = qh ? dvg + (int64_t)kj * p.ss[BDV] : dkg + (int64_t)kj * p.ss[BDK];
+        const float f = qh ? 1.f : p.scale;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                float x[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int r = 4 * g4 + e;
+                    x[e] = ((qh ? dv_acc[db][r] : dk_acc[db][r]) + part[64 * (16 * db + r) + (wave ^ 1) * (NDB * 1024)]) * f;
+                }
+                *(u32x2_t *)(row + 32 * db + 8 * g4 + 4 * hi) = u32x2_t{E::pack2(x[0], x[1]), E::pack2(x[2], x[3])};
+            }
+        return;
     }
 
     // ---- epilogue: dk = scale * dK^T, dv = dV^T; lane = key column ----

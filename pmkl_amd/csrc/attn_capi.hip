@@ -43,6 +43,23 @@ PMKL_W64_EXTERN(_Float16, false)
 #undef PMKL_W64_EXTERN
 extern template __global__ void attn_fwd_w64_kernel<__bf16, 64, true, 1, 4>(AttnParams);
 extern template __global__ void attn_fwd_w64_kernel<_Float16, 64, true, 1, 4>(AttnParams);
+extern template __global__ void attn_fwd_w64_kernel<__bf16, 128, true, 1, 4>(AttnParams);
+extern template __global__ void attn_fwd_w64_kernel<_Float16, 128, true, 1, 4>(AttnParams);
+extern template __global__ void attn_fwd_w64_kernel<__bf16, 128, false, 1, 4>(AttnParams);
+extern template __global__ void attn_fwd_w64_kernel<_Float16, 128, false, 1, 4>(AttnParams);
+// The key-split form of the 16-bit backward: attn_bwd_split_<dtype>.hip.
+#define PMKL_BWD_SPLIT_EXTERN(T, D)                                                    \
+    extern template __global__ void attn_bwd_dq_kernel<T, D, true, 2>(BwdParams);      \
+    extern template __global__ void attn_bwd_dq_kernel<T, D, false, 2>(BwdParams);     \
+    extern template __global__ void attn_bwd_dkdv_kernel<T, D, true, 2>(BwdParams);    \
+    extern template __global__ void attn_bwd_dkdv_kernel<T, D, false, 2>(BwdParams);
+PMKL_BWD_SPLIT_EXTERN(__bf16, 32)
+PMKL_BWD_SPLIT_EXTERN(__bf16, 64)
+PMKL_BWD_SPLIT_EXTERN(__bf16, 128)
+PMKL_BWD_SPLIT_EXTERN(_Float16, 32)
+PMKL_BWD_SPLIT_EXTERN(_Float16, 64)
+PMKL_BWD_SPLIT_EXTERN(_Float16, 128)
+#undef PMKL_BWD_SPLIT_EXTERN
 }  // namespace pmkl_amd
 
 namespace {
@@ -155,8 +172,8 @@ KernelChoice pick_w32(bool causal) {
                    : (kernel_fn)pmkl_amd::attn_fwd_w64_kernel<T, D, false, 1, 8>,
             512, 256, 1, "attn_fwd_w64_kernel", 1, 8};
 }
-// Two 128-row workgroups per CU for small causal head_dim-64 problems unless
-// PMKL_ATTN_SPLIT=0 (read once).
+// 128-row workgroups of the 64-row kernel for problems with few work items
+// unless PMKL_ATTN_SPLIT=0 (read once).
 bool split_enabled() {
     static const bool on = [] {
         const char *e = getenv("PMKL_ATTN_SPLIT");
@@ -173,14 +190,23 @@ bool f32split_enabled() {
     return on;
 }
 
-// split: causal head_dim 64 with fewer 256-row work items than two per CU
-// runs two 128-row workgroups per CU instead (measured same-box: B1 H8 S8192
-// 129 -> 102 us, B3 H5 S700 16.4 -> 13.0 us; equal at C2, 1-2% slower with
-// two or more 256-row items per CU).
+// split: 128-row workgroups of four waves for problems with few work items.
+// Causal head_dim 64 with fewer 256-row work items than two per CU: two of them
+// per CU (measured same-box: B1 H8 S8192 129 -> 102 us, B3 H5 S700 16.4 -> 13.0
+// us; equal at C2, 1-2% slower with two or more 256-row items per CU).
+// Head_dim 128 (one per CU) with at most half as many items as CUs, and causal
+// rows from 1,024 on up to one item per CU, where the longest item sets the
+// time (us without / with, by items: full S2047 128: 47.8 / 41.1, 256: 68.3 /
+// 77.8; causal S512 128: 19.5 / 15.5, 256: 22.0 / 23.5; causal S2047 128: 45.3 /
+// 35.2, 256: 51.3 / 46.9; causal S1024 256: 32.3 / 30.3).
 template <typename T>
 KernelChoice pick_w32(int64_t D, bool causal, bool split) {
     if (D == 64 && causal && split)
         return {(kernel_fn)pmkl_amd::attn_fwd_w64_kernel<T, 64, true, 1, 4>, 256, 128, 2, "attn_fwd_w64_kernel", 1, 4};
+    if (D == 128 && split)
+        return {causal ? (kernel_fn)pmkl_amd::attn_fwd_w64_kernel<T, 128, true, 1, 4>
+                       : (kernel_fn)pmkl_amd::attn_fwd_w64_kernel<T, 128, false, 1, 4>,
+                256, 128, 1, "attn_fwd_w64_kernel", 1, 4};
     return D == 64 ? pick_w32<T, 64>(causal) : pick_w32<T, 128>(causal);
 }
 
@@ -297,15 +323,19 @@ struct BwdKernels {
     int dkdv_threads, dkdv_rows;
 };
 
-template <typename T, int D>
+template <typename T, int D, int KS>
 BwdKernels pick_bwd(bool causal) {
-    using TQ = pmkl_amd::BwdTile<T, D, pmkl_amd::bwd_waves_dq<D>()>;
-    using TK = pmkl_amd::BwdTile<T, D, pmkl_amd::bwd_waves_dkdv<D>()>;
+    using TQ = pmkl_amd::BwdTile<T, D, pmkl_amd::bwd_waves_dq<D>(), KS>;
+    using TK = pmkl_amd::BwdTile<T, D, pmkl_amd::bwd_waves_dkdv<D>(), KS>;
     if (causal)
-        return {pmkl_amd::attn_bwd_dq_kernel<T, D, true>, pmkl_amd::attn_bwd_dkdv_kernel<T, D, true>, TQ::THREADS,
-                TQ::ROWS, TK::THREADS, TK::ROWS};
-    return {pmkl_amd::attn_bwd_dq_kernel<T, D, false>, pmkl_amd::attn_bwd_dkdv_kernel<T, D, false>, TQ::THREADS,
-            TQ::ROWS, TK::THREADS, TK::ROWS};
+        return {pmkl_amd::attn_bwd_dq_kernel<T, D, true, KS>, pmkl_amd::attn_bwd_dkdv_kernel<T, D, true, KS>,
+                TQ::THREADS, TQ::ROWS, TK::THREADS, TK::ROWS};
+    return {pmkl_amd::attn_bwd_dq_kernel<T, D, false, KS>, pmkl_amd::attn_bwd_dkdv_kernel<T, D, false, KS>,
+            TQ::THREADS, TQ::ROWS, TK::THREADS, TK::ROWS};
+}
+template <typename T, int D>
+BwdKernels pick_bwd(bool causal, bool split) {
+    return split ? pick_bwd<T, D, 2>(causal) : pick_bwd<T, D, 1>(causal);
 }
 
 template <int D>
@@ -316,15 +346,53 @@ BwdKernels pick_bwd_f32(bool causal) {
     return {pmkl_amd::attn_bwd_f32_dq_kernel<D, false>, pmkl_amd::attn_bwd_f32_dkdv_kernel<D, false>, T, R, T, R};
 }
 
-BwdKernels select_bwd(int32_t dt, int64_t d, bool causal) {
+// PMKL_ATTN_BWDSPLIT=0: the split form of the 16-bit backward never, =1
+// wherever it applies (read once); -1 if unset.
+int bwd_split_mode() {
+    static const int v = [] {
+        const char *e = getenv("PMKL_ATTN_BWDSPLIT");
+        return e ? (atoi(e) == 1 ? 1 : 0) : -1;
+    }();
+    return v;
+}
+// Split form of the 16-bit backward (attn_bwd_kernels.hpp, KS = 2): where the
+// 128-row workgroups leave CUs idle, or are so few that the longest causal one
+// sets the time.  It costs a quarter more once they fill the chip.  Measured
+// without / with it, us per backward call (bf16, without O), by 128-row workgroups:
+//   head_dim 128 full    128: 152.9 / 117.0 (S 2047), 36.7 / 29.7 (S 200);  256: 174 / 218, 38.9 / 55.2
+//                causal  128: 156.9 / 107.2;  256: 158 / 131 (S 2047), 90.1 / 83.6 (S 1024), 57.7 / 61.7 (S 512);
+//                        512: 196 / 252
+//   head_dim 64  full    128: 99.3 / 70.4;  256: 105.7 / 105.0 (S 2047), 24.0 / 25.5 (S 200)
+//                causal  256: 104.3 / 79.7 (S 2047), 23.9 / 22.2 (S 200);  512: 122 / 121 (S 2047), 46.1 / 54.1 (S 512)
+//   head_dim 32  full    256: 75.4 / 65.5 (S 2047), 23.3 / 21.6 (S 200);  512: 112 / 121
+//                causal  256: 78.9 / 53.7;  512: 82.6 / 72.8 (S 2047), 47.1 / 42.9 (S 1024);  1,024: 121 / 132
+bool bwd_split(const pmkl_attn_bwd_args *a) {
+    const int64_t S = a->seq_len, D = a->head_dim;
+    // its dK/dV pass addresses 128 rows of Q and dout by one 32-bit buffer range
+    if (std::max(a->q_strides[2], a->dout_strides[2]) * 2 * 128 >= (1LL << 31)) return false;
+    if (bwd_split_mode() >= 0) return bwd_split_mode() == 1;
+    const bool long_causal = a->is_causal != 0 && S >= 1024;
+    const int64_t cus = cu_count(), groups = a->batch * a->heads * ((S + 127) / 128);
+    const int64_t most = D == 128  ? (long_causal ? cus : cus / 2)
+                         : D == 64 ? (a->is_causal != 0 ? cus : cus / 2)
+                                   : (long_causal ? 2 * cus : cus);
+    return groups <= most;
+}
+
+BwdKernels select_bwd(const pmkl_attn_bwd_args *a) {
+    const int32_t dt = a->dtype;
+    const int64_t d = a->head_dim;
+    const bool causal = a->is_causal != 0;
     if (dt == PMKL_DTYPE_BF16) {
-        if (d == 32) return pick_bwd<__bf16, 32>(causal);
-        if (d == 64) return pick_bwd<__bf16, 64>(causal);
-        if (d == 128) return pick_bwd<__bf16, 128>(causal);
+        const bool split = bwd_split(a);
+        if (d == 32) return pick_bwd<__bf16, 32>(causal, split);
+        if (d == 64) return pick_bwd<__bf16, 64>(causal, split);
+        if (d == 128) return pick_bwd<__bf16, 128>(causal, split);
     } else if (dt == PMKL_DTYPE_F16) {
-        if (d == 32) return pick_bwd<_Float16, 32>(causal);
-        if (d == 64) return pick_bwd<_Float16, 64>(causal);
-        if (d == 128) return pick_bwd<_Float16, 128>(causal);
+        const bool split = bwd_split(a);
+        if (d == 32) return pick_bwd<_Float16, 32>(causal, split);
+        if (d == 64) return pick_bwd<_Float16, 64>(causal, split);
+        if (d == 128) return pick_bwd<_Float16, 128>(causal, split);
     } else if (dt == PMKL_DTYPE_F32) {
         if (d == 32) return pick_bwd_f32<32>(causal);
         if (d == 64) return pick_bwd_f32<64>(causal);
@@ -381,7 +449,7 @@ int check_bwd(const pmkl_attn_bwd_args *a, bool *empty) {
     const size_t ml_es = dtype_size(a->ml_dtype);
     PMKL_REQUIRE((uintptr_t)a->m % ml_es == 0 && (uintptr_t)a->l % ml_es == 0, PMKL_EINVAL,
                  "m / l must be aligned to their element size");
-    const BwdKernels kc = select_bwd(a->dtype, D, a->is_causal != 0);
+    const BwdKernels kc = select_bwd(a);
     PMKL_REQUIRE(kc.dq != nullptr, PMKL_EUNSUPPORTED, "no backward kernel for dtype %d head_dim %lld",
                  (int)a->dtype, (long long)D);
     const int64_t nq = (S + kc.dq_rows - 1) / kc.dq_rows, nk = (S + kc.dkdv_rows - 1) / kc.dkdv_rows;
@@ -397,7 +465,7 @@ int check_bwd(const pmkl_attn_bwd_args *a, bool *empty) {
 // nothing in it needs clearing.
 int launch_bwd(const pmkl_attn_bwd_args *a, float *ws, void *stream) {
     const int64_t B = a->batch, H = a->heads, S = a->seq_len, D = a->head_dim;
-    const BwdKernels kc = select_bwd(a->dtype, D, a->is_causal != 0);
+    const BwdKernels kc = select_bwd(a);
     const int64_t nq = (S + kc.dq_rows - 1) / kc.dq_rows, nk = (S + kc.dkdv_rows - 1) / kc.dkdv_rows;
     const int64_t gq = nq * B * H, gk = nk * B * H;
 
@@ -550,14 +618,18 @@ int plan_fwd(const pmkl_attn_fwd_args *a, FwdPlan *pl) {
     const int waves = small128 && !waves16_env() ? 4 : waves16(D, S, causal);
     const bool resident = !w64 && a->dtype != PMKL_DTYPE_F32 && waves == 8 &&
                           (S + 63) / 64 <= resident_tiles(D) && resident_enabled();
-    const bool split = w32 && D == 64 && causal && split_enabled() &&
-                       B * H * ((S + 255) / 256) < 2 * (int64_t)cu_count();
+    const int64_t items = B * H * ((S + 255) / 256);
+    const bool split = w32 && split_enabled() &&
+                       (D == 64 ? causal && items < 2 * (int64_t)cu_count()
+                                : items <= (causal && S >= 1024 ? cu_count() : cu_count() / 2));
     // fp32: 32-row workgroups whose four waves split the key tiles, at every
     // size (measured against the 128-row kernel, us: B1 H4 S128 D64 6.3 / 17.1,
     // B4 H16 S1024 D64 96 / 126, B2 H4 S2048 D128 144 / 326, B1 H32 S4096 D128
     // 1,109 / 1,357, B256 H8 S20 D64 19.1 / 21.4).  The 128-row kernel is left
-    // for PMKL_ATTN_F32SPLIT=0 and for a device whose CU count cannot be read.
-    const bool f32split = a->dtype == PMKL_DTYPE_F32 && f32split_enabled() && cu_count() > 0;
+    // for PMKL_ATTN_F32SPLIT=0, for a device whose CU count cannot be read, and
+    // where 32-row workgroups of 256 threads would pass a launch's 2^32 threads.
+    const bool f32split = a->dtype == PMKL_DTYPE_F32 && f32split_enabled() && cu_count() > 0 &&
+                          B * H * ((S + 31) / 32) < (1LL << 24);
     const KernelChoice kc = w32        ? (bf ? pick_w32<__bf16>(D, causal, split) : pick_w32<_Float16>(D, causal, split))
                             : f32split ? pick32split(D, causal)
                                        : select_kernel(a->dtype, D, causal, w64, waves, resident);

@@ -8,6 +8,7 @@
 namespace pmkl_amd {
 template __global__ void attn_fwd_w64_kernel<__bf16, 64, false, 1, 8>(AttnParams);
 template __global__ void attn_fwd_w64_kernel<__bf16, 128, false, 1, 8>(AttnParams);
+template __global__ void attn_fwd_w64_kernel<__bf16, 128, false, 1, 4>(AttnParams);
 template __global__ void attn_fwd_w64_kernel<__bf16, 32, false, 2, 4>(AttnParams);
 template __global__ void attn_fwd_w64_kernel<__bf16, 64, false, 2, 4>(AttnParams);
 template __global__ void attn_fwd_w64_kernel<__bf16, 128, false, 2, 4>(AttnParams);

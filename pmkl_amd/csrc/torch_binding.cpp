@@ -364,7 +364,20 @@ public:
         const auto saved = ctx->get_saved_variables();
         const at::Tensor &q = saved[0], &out = saved[3];
         // without a gradient of out its zeros, as the Python function sees them
-        const at::Tensor dout = grads[0].defined() ? grads[0] : at::zeros_like(out);
+        at::Tensor dout = grads[0].defined() ? grads[0] : at::zeros_like(out);
+        // Saved-tensor hooks may hand back anything; the kernels get pointers.
+        bool same = q.dim() == 4 && q.is_cuda();
+        for (const at::Tensor &t : {saved[1], saved[2], out, dout})
+            same = same && t.sizes() == q.sizes() && t.scalar_type() == q.scalar_type() && t.device() == q.device();
+        for (const at::Tensor &t : {saved[4], saved[5]})
+            same = same && t.sizes() == q.sizes().slice(0, 3) && t.device() == q.device();
+        TORCH_CHECK(same, "fused_self_attention: a saved tensor came back with another shape, dtype or device");
+        // The stride of a dimension of size 1 is never used and may hold
+        // anything; the checks on strides would refuse it.
+        std::vector<int64_t> st = dout.strides().vec();
+        for (int i = 0; i < 3; ++i)
+            if (dout.size(i) == 1) st[i] = i < 2 ? 0 : dout.size(3);
+        if (dout.strides() != at::IntArrayRef(st)) dout = dout.as_strided(dout.sizes(), st);
         at::Tensor dq, dk, dv;
         std::tie(dq, dk, dv) = device_backward(dout, q, saved[1], saved[2], out, saved[4], saved[5],
                                                ctx->saved_data["is_causal"].toBool());

@@ -89,3 +89,31 @@ def test_side_stream(device):
     torch.cuda.current_stream().wait_stream(s)
     torch.cuda.synchronize()
     assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
+def test_gradient_strides_of_single_dimensions(device):
+    """A dimension of size 1 may carry any stride; such a gradient gives the
+    result of its contiguous copy."""
+    import torch
+    from pmkl_amd.pmkl_function import fused_self_attention
+
+    for B, H, S in ((1, 3, 40), (2, 1, 40), (1, 1, 40), (2, 3, 1)):
+        q, k, v, do = _inputs(torch.bfloat16, B=B, H=H, S=S, D=32)
+        st = [7 if n == 1 else x for n, x in zip(do.shape[:3], do.stride())] + [1]
+        odd = do.as_strided(do.shape, st)
+        a = torch.autograd.grad(fused_self_attention(q, k, v, True)[0], (q, k, v), odd)
+        b = torch.autograd.grad(fused_self_attention(q, k, v, True)[0], (q, k, v), do)
+        assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+def test_saved_tensors_that_come_back_different(device):
+    """What a saved-tensor hook returns is checked before a kernel gets its pointer."""
+    import torch
+    from pmkl_amd.pmkl_function import fused_self_attention
+
+    q, k, v, do = _inputs(torch.bfloat16)
+    for unpack in (lambda t: t[..., :1], lambda t: t.float() if t.dim() == 4 else t[..., :1], lambda t: t.cpu()):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            out = fused_self_attention(q, k, v, True)[0]
+        with pytest.raises(RuntimeError, match="came back"):
+            torch.autograd.grad(out, (q, k, v), do)
