@@ -20,13 +20,20 @@
 // a four-way split give many short, equal workgroups: the chains of dependent
 // tiles are a quarter as long as with one wave per row block, which bounds the
 // small shapes, and the long causal rows start first.
+// Hidden keys and queries must add nothing, whatever they hold.  In the products
+// over a whole tile their weight is 0, and 0 times an infinity or a NaN is a
+// NaN: a row whose sum is not finite is computed again, over its visible keys or
+// queries alone (attn_bwd_f32_rows.hpp).  The check of the sums costs 1-2% where
+// a workgroup has one round of tiles (1,024 heads of S128 D64 causal, whole
+// call, 171.8 / 176.2 us) and nothing from S1024 on; masking P, dS and the tiles
+// themselves cost 10-18% at every causal size.
 // Measured against one wave per owned row on the vector ALUs (dq / dkdv, us):
 // B4 H16 S1024 D64 causal 3,141 / 3,303 -> 132 / 180 (96 and 128 fp32 MFMAs per
 // tile: 84 and 112 us at the MFMA's 154 TFLOP/s), B2 H16 S128 D128 90 / 123 ->
 // 14 / 16 (one tile per wave: latency).
 #pragma once
 
-#include "attn_bwd_kernels.hpp"
+#include "attn_bwd_f32_rows.hpp"
 #include "attn_f32.hpp"
 
 namespace pmkl_amd {
@@ -149,8 +156,8 @@ __global__ __launch_bounds__(kF32Threads, D >= 128 ? 1 : D >= 64 ? 3 : 4) void a
     asm volatile("" ::: "memory");
     if (wave < nt) f32_put<D>(tile, acc, col, hi);
     __syncthreads();
-    f32_combine<D>(smem[0], TL::FLOATS, min(NW, nt), p.scale, bwd_head<float>(p, p.dq, BDQ, bh), q0, S,
-                       p.ss[BDQ]);
+    f32_combine<D>(smem[0], TL::FLOATS, min(NW, nt), p.scale, bwd_head<float>(p, p.dq, BDQ, bh), q0, S, p.ss[BDQ],
+                   [&](int row) { f32_dq_row<D, CAUSAL>(p, bh, row); });
 }
 
 template <int D, bool CAUSAL>
@@ -240,11 +247,12 @@ __global__ __launch_bounds__(kF32Threads, D >= 128 ? 1 : D >= 64 ? 3 : 4) void a
     asm volatile("" ::: "memory");
     if (t0 + wave < nq) f32_put<D>(tile, dk_acc, col, hi);
     __syncthreads();
-    f32_combine<D>(smem[0], TL::FLOATS, n, p.scale, bwd_head<float>(p, p.dk, BDK, bh), k0, S, p.ss[BDK]);
+    auto redo = [&](int row) { f32_dkdv_row<D, CAUSAL>(p, bh, row); };
+    f32_combine<D>(smem[0], TL::FLOATS, n, p.scale, bwd_head<float>(p, p.dk, BDK, bh), k0, S, p.ss[BDK], redo);
     __syncthreads();
     if (t0 + wave < nq) f32_put<D>(tile, dv_acc, col, hi);
     __syncthreads();
-    f32_combine<D>(smem[0], TL::FLOATS, n, 1.f, bwd_head<float>(p, p.dv, BDV, bh), k0, S, p.ss[BDV]);
+    f32_combine<D>(smem[0], TL::FLOATS, n, 1.f, bwd_head<float>(p, p.dv, BDV, bh), k0, S, p.ss[BDV], redo);
 }
 
 }  // namespace pmkl_amd

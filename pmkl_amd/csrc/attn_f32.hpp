@@ -166,18 +166,47 @@ __device__ __forceinline__ void f32_put(float *part, const f32x16_t (&acc)[D / 3
 }
 
 // Adds the partials of the first n waves (wave_floats apart) and stores
-// scale times the sum to rows r0 .. of out, whole rows at a time.
-template <int D>
+// scale times the sum to rows r0 .. of out, whole rows at a time.  Then
+// redo(row) for each row whose sum is not finite, by the one wave that stored
+// it (nothing is checked with the default).
+struct F32Keep {};
+template <int D, typename Redo = F32Keep>
 __device__ __forceinline__ void f32_combine(const float *part, int wave_floats, int n, float scale, float *out,
-                                                int r0, int S, int ss) {
+                                                int r0, int S, int ss, Redo redo = {}) {
     using TL = F32Tile<D>;
-    constexpr int THREADS = kF32Threads;
+    constexpr int THREADS = kF32Threads, SLOTS = kF32Rows * TL::CPR / THREADS;
+    const int ch = threadIdx.x % TL::CPR;
+    auto row_of = [](int i) __attribute__((always_inline)) { return (i * THREADS + (int)threadIdx.x) / TL::CPR; };
+    auto sum_of = [&](int i) __attribute__((always_inline)) {
+        f32x4_t sum = *(const f32x4_t *)(part + row_of(i) * TL::LD + 4 * ch);
+        for (int w = 1; w < n; ++w) sum += *(const f32x4_t *)(part + w * wave_floats + row_of(i) * TL::LD + 4 * ch);
+        return sum * scale;
+    };
+    auto add_zeros = [](float z, const f32x4_t &x) __attribute__((always_inline)) {   // NaN if x is not finite
 #pragma unroll
-    for (int i = 0; i < kF32Rows * TL::CPR / THREADS; ++i) {
-        const int sl = i * THREADS + (int)threadIdx.x, row = sl / TL::CPR, ch = sl % TL::CPR;
-        f32x4_t sum = *(const f32x4_t *)(part + row * TL::LD + 4 * ch);
-        for (int w = 1; w < n; ++w) sum += *(const f32x4_t *)(part + w * wave_floats + row * TL::LD + 4 * ch);
-        if (r0 + row < S) *(f32x4_t *)(out + (int64_t)(r0 + row) * ss + 4 * ch) = sum * scale;
+        for (int e = 0; e < 4; ++e) z = __builtin_fmaf(x[e], 0.f, z);
+        return z;
+    };
+    float z = 0.f;
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+        const f32x4_t sum = sum_of(i);
+        if constexpr (!std::is_same_v<Redo, F32Keep>) z = add_zeros(z, sum);
+        if (r0 + row_of(i) < S) *(f32x4_t *)(out + (int64_t)(r0 + row_of(i)) * ss + 4 * ch) = sum;
+    }
+    if constexpr (!std::is_same_v<Redo, F32Keep>) {
+        if (__builtin_amdgcn_ballot_w64(z != z) == 0) return;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");   // other lanes of the wave store the rows again
+        constexpr uint64_t lanes = (1ull << TL::CPR) - 1;    // a row's, from its first
+#pragma unroll 1
+        for (int i = 0; i < SLOTS; ++i) {
+            const float zi = add_zeros(0.f, sum_of(i));
+            const uint64_t bad = __builtin_amdgcn_ballot_w64(zi != zi && r0 + row_of(i) < S);
+            const int first = __builtin_amdgcn_readfirstlane(row_of(i));
+#pragma unroll 1
+            for (int w = 0; w < 64 / TL::CPR; ++w)
+                if (bad >> (w * TL::CPR) & lanes) redo(r0 + first + w);
+        }
     }
 }
 
