@@ -33,7 +33,7 @@ SCC_WRITE = re.compile(
 SCC_READ = re.compile(r"^(s_cselect|s_cbranch_scc|s_addc_u32|s_subb_u32|s_cmov)")
 
 
-# The head_dim-128 backward kernels, instantiated explicitly.
+# The head_dim-128 backward kernels in both forms, instantiated explicitly.
 BWD_TU = """#include <hip/hip_runtime.h>
 #include "attn_bwd_kernels.hpp"
 namespace pmkl_amd {
@@ -41,6 +41,10 @@ template __global__ void attn_bwd_dq_kernel<__bf16, 128, true>(BwdParams);
 template __global__ void attn_bwd_dq_kernel<__bf16, 128, false>(BwdParams);
 template __global__ void attn_bwd_dq_kernel<_Float16, 128, true>(BwdParams);
 template __global__ void attn_bwd_dkdv_kernel<__bf16, 128, true>(BwdParams);
+template __global__ void attn_bwd_dq_kernel<__bf16, 128, true, 2>(BwdParams);
+template __global__ void attn_bwd_dq_kernel<__bf16, 128, false, 2>(BwdParams);
+template __global__ void attn_bwd_dq_kernel<_Float16, 128, true, 2>(BwdParams);
+template __global__ void attn_bwd_dkdv_kernel<__bf16, 128, true, 2>(BwdParams);
 }
 """
 
@@ -104,7 +108,7 @@ def test_no_scc_read_across_lds_dma(asm_lines):
 
 def test_backward_kernels_compiled_with_lds_dma(bwd_asm_lines):
     kernels = [l for l in bwd_asm_lines if re.match(r"^_ZN8pmkl_amd(18attn_bwd_dq|20attn_bwd_dkdv)_kernel.*:$", l)]
-    assert len(kernels) == 4, kernels
+    assert len(kernels) == 8, kernels
     assert sum(1 for l in bwd_asm_lines if l.startswith("buffer_load_dwordx4") and l.endswith(" lds")) > 0
 
 
