@@ -29,7 +29,8 @@ def main() -> int:
               (2, 2, 200, 32, "fp16", True), (1, 5, 1000, 128, "bf16", True), (3, 2, 256, 64, "fp16", True),
               (2, 2, 128, 128, "bf16", False), (1, 2, 129, 128, "fp16", True), (2, 1, 384, 128, "bf16", False),
               (1, 4, 128, 64, "fp32", True), (2, 1, 300, 128, "fp32", False), (1, 2, 33, 32, "fp32", True),
-              (2, 8, 300, 64, "bf16", True)]
+              (2, 8, 300, 64, "bf16", True), (1, 150, 257, 128, "bf16", False),   # more items than the split takes
+              (1, 2, 400, 128, "fp16", False)]
     env = {k: v for k, v in os.environ.items() if k.startswith("PMKL_ATTN")}
     names = []
     for i, (B, H, S, D, dt, causal) in enumerate(shapes):

@@ -27,7 +27,7 @@ SETTINGS = [
     {"PMKL_ATTN_W64": "0", "PMKL_ATTN_WAVES": "4"},  # the 4-wave MFMA kernel everywhere
     {"PMKL_ATTN_NOXCD": "1"},                        # plain (head, tile) work order
     {"PMKL_ATTN_RESIDENT": "0"},                     # short sequences on the streaming 8-wave kernel
-    {"PMKL_ATTN_SPLIT": "0"},                        # small causal head_dim-64 problems on 256-row workgroups
+    {"PMKL_ATTN_SPLIT": "0"},                        # the 64-row kernel's small problems on 256-row workgroups
     {"PMKL_ATTN_F32SPLIT": "0"},                     # small fp32 problems on the 128-row fp32 kernel
 ]
 
@@ -60,9 +60,11 @@ def _expect_kernels(setting, shapes, names, base):
     sixteen = [(s, n) for s, n in zip(shapes, names) if s[4] != "fp32"]
     key = tuple(sorted(setting.items()))
     if key == (("PMKL_ATTN_W32", "0"),):
-        for s, n, b in zip(shapes, names, base):
-            if b.startswith("attn_fwd_w64_kernel") and ", 1, 8>" in b:
-                assert n.startswith("attn_fwd_w64_kernel") and ", 2, 4>" in n, (s, n, b)
+        eight = [(s, n, b) for s, n, b in zip(shapes, names, base)
+                 if b.startswith("attn_fwd_w64_kernel") and ", 1, 8>" in b]
+        assert any(s[3] == 128 for s, _, _ in eight), base
+        for s, n, b in eight:
+            assert n.startswith("attn_fwd_w64_kernel") and ", 2, 4>" in n, (s, n, b)
     elif key == (("PMKL_ATTN_W64", "0"),):
         assert not any(n.startswith("attn_fwd_w64_kernel") for _, n in sixteen), names
     elif key == (("PMKL_ATTN_W64", "1"),):
@@ -78,7 +80,10 @@ def _expect_kernels(setting, shapes, names, base):
         assert not any(n.startswith("attn_fwd_mfma16_kernel") and not n.split(">")[0].endswith(", 0")
                        for n in names), names
     elif key == (("PMKL_ATTN_SPLIT", "0"),):
-        assert not any(", 64, causal, 1, 4>" in n for n in names), names
+        assert not any(", 1, 4>" in n for n in names), names
+        for D in (64, 128):
+            assert any(f", {D}, causal, 1, 4>" in b for b in base), base
+        assert any(", 128, full, 1, 4>" in b for b in base), base
     elif key == (("PMKL_ATTN_F32SPLIT", "0"),):
         assert not any(n.startswith("attn_fwd_f32_split_kernel") for n in names), names
     else:
