@@ -176,6 +176,13 @@ int pmkl_attn_bwd(const pmkl_attn_bwd_args *args, void *stream);
 /* 1 if a backward kernel is compiled for (dtype, head_dim), else 0. */
 int pmkl_attn_bwd_supported(int32_t dtype, int64_t head_dim);
 
+/* The two kernels pmkl_attn_bwd would launch for these arguments (the workspace
+ * is not looked at), with their launch shapes, e.g.
+ * "attn_bwd_dq_kernel<bf16, 64, causal, 2> grid 32 x 256, attn_bwd_dkdv_kernel<bf16, 64, causal, 2> grid 32 x 256";
+ * otherwise as pmkl_attn_fwd_kernel_name, with a string of its own.  An addition
+ * to ABI version 5. */
+const char *pmkl_attn_bwd_kernel_name(const pmkl_attn_bwd_args *args);
+
 /* Largest batch * heads * seq_len that pmkl_attn_bwd_noalloc accepts. */
 #define PMKL_ATTN_BWD_NOALLOC_MAX_ROWS 1048576
 

@@ -32,6 +32,7 @@ EXPORTED_SYMBOLS = (
     "pmkl_attn_fwd_supported",
     "pmkl_attn_bwd_workspace_size",
     "pmkl_attn_bwd",
+    "pmkl_attn_bwd_kernel_name",
     "pmkl_attn_bwd_supported",
     "pmkl_attn_bwd_noalloc",
     "pmkl_last_error",
@@ -154,6 +155,8 @@ def load() -> ctypes.CDLL:
     lib.pmkl_abi_version.restype = ctypes.c_int
     lib.pmkl_attn_bwd_workspace_size.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64]
     lib.pmkl_attn_bwd_workspace_size.restype = ctypes.c_uint64
+    lib.pmkl_attn_bwd_kernel_name.argtypes = [ctypes.POINTER(AttnBwdArgs)]
+    lib.pmkl_attn_bwd_kernel_name.restype = ctypes.c_char_p
     lib.pmkl_attn_bwd.argtypes = [ctypes.POINTER(AttnBwdArgs), ctypes.c_void_p]
     lib.pmkl_attn_bwd.restype = ctypes.c_int
     lib.pmkl_attn_bwd_noalloc.argtypes = [ctypes.POINTER(AttnBwdArgs), ctypes.c_void_p]
@@ -213,6 +216,13 @@ def make_args(q, k, v, o, m, l, *, dtype: int, ml_dtype: int | None = None, batc
 def attn_bwd_raw(args: AttnBwdArgs, stream: int | None = None) -> int:
     """Call pmkl_attn_bwd; returns the status code."""
     return load().pmkl_attn_bwd(ctypes.byref(args), ctypes.c_void_p(stream or 0))
+
+
+def attn_bwd_kernel_name(args: AttnBwdArgs) -> str | None:
+    """The two kernels (and launch shapes) pmkl_attn_bwd would launch for args;
+    None where the call would fail (last_error() says why)."""
+    name = load().pmkl_attn_bwd_kernel_name(ctypes.byref(args))
+    return None if name is None else name.decode()
 
 
 def attn_bwd_noalloc_raw(args: AttnBwdArgs, stream: int | None = None) -> int:

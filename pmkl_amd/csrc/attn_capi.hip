@@ -321,6 +321,8 @@ struct BwdKernels {
     bwd_kernel_fn dq, dkdv;
     int dq_threads, dq_rows;       // threads and owned rows per workgroup
     int dkdv_threads, dkdv_rows;
+    const char *family = "";       // names them for pmkl_attn_bwd_kernel_name: <family>_dq_kernel, <family>_dkdv_kernel
+    int ks = -1;                   // template parameter after the mask, -1 if none
 };
 
 template <typename T, int D, int KS>
@@ -329,9 +331,9 @@ BwdKernels pick_bwd(bool causal) {
     using TK = pmkl_amd::BwdTile<T, D, pmkl_amd::bwd_waves_dkdv<D>(), KS>;
     if (causal)
         return {pmkl_amd::attn_bwd_dq_kernel<T, D, true, KS>, pmkl_amd::attn_bwd_dkdv_kernel<T, D, true, KS>,
-                TQ::THREADS, TQ::ROWS, TK::THREADS, TK::ROWS};
+                TQ::THREADS, TQ::ROWS, TK::THREADS, TK::ROWS, "attn_bwd", KS};
     return {pmkl_amd::attn_bwd_dq_kernel<T, D, false, KS>, pmkl_amd::attn_bwd_dkdv_kernel<T, D, false, KS>,
-            TQ::THREADS, TQ::ROWS, TK::THREADS, TK::ROWS};
+            TQ::THREADS, TQ::ROWS, TK::THREADS, TK::ROWS, "attn_bwd", KS};
 }
 template <typename T, int D>
 BwdKernels pick_bwd(bool causal, bool split) {
@@ -342,8 +344,10 @@ template <int D>
 BwdKernels pick_bwd_f32(bool causal) {
     constexpr int T = pmkl_amd::kF32Threads, R = pmkl_amd::kF32Rows;
     if (causal)
-        return {pmkl_amd::attn_bwd_f32_dq_kernel<D, true>, pmkl_amd::attn_bwd_f32_dkdv_kernel<D, true>, T, R, T, R};
-    return {pmkl_amd::attn_bwd_f32_dq_kernel<D, false>, pmkl_amd::attn_bwd_f32_dkdv_kernel<D, false>, T, R, T, R};
+        return {pmkl_amd::attn_bwd_f32_dq_kernel<D, true>, pmkl_amd::attn_bwd_f32_dkdv_kernel<D, true>, T, R, T, R,
+                "attn_bwd_f32"};
+    return {pmkl_amd::attn_bwd_f32_dq_kernel<D, false>, pmkl_amd::attn_bwd_f32_dkdv_kernel<D, false>, T, R, T, R,
+            "attn_bwd_f32"};
 }
 
 // PMKL_ATTN_BWDSPLIT=0: the split form of the 16-bit backward never, =1
@@ -718,6 +722,24 @@ const char *pmkl_attn_fwd_kernel_name(const pmkl_attn_fwd_args *a) {
     else
         snprintf(name, sizeof(name), "%s<%lld, %s> grid %lld x %d%s", pl.kc.family, (long long)a->head_dim, mask,
                  (long long)pl.grid, pl.kc.threads, order);
+    return name;
+}
+
+const char *pmkl_attn_bwd_kernel_name(const pmkl_attn_bwd_args *a) {
+    pmkl_capi::g_err[0] = '\0';
+    static thread_local char name[320];
+    bool empty = false;
+    if (check_bwd(a, &empty) != PMKL_OK) return nullptr;
+    if (empty) return "none";
+    const BwdKernels kc = select_bwd(a);
+    const char *dt = a->dtype == PMKL_DTYPE_BF16 ? "bf16, " : a->dtype == PMKL_DTYPE_F16 ? "fp16, " : "";
+    char args[64], ks[16] = "";
+    if (kc.ks >= 0) snprintf(ks, sizeof(ks), ", %d", kc.ks);
+    snprintf(args, sizeof(args), "<%s%lld, %s%s>", dt, (long long)a->head_dim, a->is_causal ? "causal" : "full", ks);
+    const int64_t BH = a->batch * a->heads;
+    snprintf(name, sizeof(name), "%s_dq_kernel%s grid %lld x %d, %s_dkdv_kernel%s grid %lld x %d", kc.family, args,
+             (long long)((a->seq_len + kc.dq_rows - 1) / kc.dq_rows * BH), kc.dq_threads, kc.family, args,
+             (long long)((a->seq_len + kc.dkdv_rows - 1) / kc.dkdv_rows * BH), kc.dkdv_threads);
     return name;
 }
 

@@ -1,0 +1,55 @@
+"""Child-process check of the 16-bit backward's forms (run by
+tests/test_bwd_forms_gpu.py with PMKL_ATTN_BWDSPLIT set; the library reads it
+once per process): the cases of test_attn_bwd_gpu.py on the form that the
+switch pins, and more of them where that form can go wrong.  Exits 0 when all
+pass."""
+from __future__ import annotations
+
+import os
+import sys
+from pathlib import Path
+
+ROOT = Path(__file__).resolve().parent.parent
+sys.path.insert(0, str(ROOT))
+
+
+def main() -> int:
+    import torch
+
+    import pmkl_amd
+    from tests import test_attn_bwd_gpu as t
+
+    form = ", 2>" if os.environ["PMKL_ATTN_BWDSPLIT"] == "1" else ", 1>"
+    raw, launched = pmkl_amd.capi.attn_bwd_raw, set()
+
+    def named(args, stream=None):   # every backward call of the cases below names its kernels first
+        name = pmkl_amd.capi.attn_bwd_kernel_name(args)
+        assert name.count(form) == 2, name
+        launched.add(name.split(" grid")[0])
+        return raw(args, stream)
+
+    pmkl_amd.capi.attn_bwd_raw = named
+    dev = torch.device("cuda:0")
+    for dtype in ("bf16", "fp16"):
+        for D in (32, 64, 128):
+            for causal in (True, False):
+                t.test_bwd_small_shapes_vs_oracle(dev, dtype, D, causal)
+                # odd and even counts of 64-row tiles, more than two per workgroup
+                for B, H, S in ((1, 1, 321), (1, 2, 449), (1, 1, 700)):
+                    tag = f"{dtype} B{B} H{H} S{S} D{D} causal={causal}"
+                    t._say(f"case {tag}")
+                    got, ref, _ = t._run(B, H, S, D, dtype, causal, seed=9500 + S, ml_dtype=torch.float32)
+                    t._check(got, ref, dtype, tag)
+            t.test_bwd_strided_views_without_copies(dev, dtype, D)
+            if D > 32:
+                t.test_bwd_with_forward_output(dev, dtype, D)
+        for causal in (True, False):
+            t.test_bwd_float_ml_from_64_row_kernel(dev, dtype, causal)
+    t.test_bwd_larger_heads_sampled(dev)
+    t.test_bwd_closed_form_constant_v(dev)
+    assert len(launched) == 12, launched   # dtypes x head_dims x masks
+    return 0
+
+
+if __name__ == "__main__":
+    sys.exit(main())

@@ -312,3 +312,21 @@ def test_kernel_name_query():
     # fp32 with the CU count unknown (no device): the 128-row fp32 kernel
     name = capi.attn_fwd_kernel_name(_args(dtype=capi.PMKL_DTYPE_F32, ml_dtype=capi.PMKL_DTYPE_F32, seq_len=300))
     assert name == "attn_fwd_f32_kernel<64, causal> grid 6 x 256", name
+
+
+def test_backward_kernel_name_query():
+    """pmkl_attn_bwd_kernel_name names the two kernels pmkl_attn_bwd would
+    launch, or returns NULL with the same error text where the call would fail."""
+    def name(dtype=capi.PMKL_DTYPE_BF16, S=300, D=64, causal=True, **kw):
+        return capi.attn_bwd_kernel_name(capi.make_bwd_args(*(range(0x1000, 0xb000, 0x1000)), 0, 0, dtype=dtype,
+                                                            batch=1, heads=2, seq_len=S, head_dim=D, is_causal=causal,
+                                                            **kw))
+
+    assert name(D=80) is None and "head_dim 80" in capi.last_error()
+    assert name(strides={"dq": (0, 64, 64)}) is None and "overlap" in capi.last_error()
+    assert name(S=0) == "none"
+    # no device, so no CU count: the 128-row form
+    assert name() == ("attn_bwd_dq_kernel<bf16, 64, causal, 1> grid 6 x 256, "
+                      "attn_bwd_dkdv_kernel<bf16, 64, causal, 1> grid 6 x 256")
+    assert name(dtype=capi.PMKL_DTYPE_F32, D=128, causal=False) == (
+        "attn_bwd_f32_dq_kernel<128, full> grid 20 x 256, attn_bwd_f32_dkdv_kernel<128, full> grid 20 x 256")
