@@ -157,7 +157,7 @@ __global__ __launch_bounds__(kF32Threads, D >= 128 ? 1 : D >= 64 ? 3 : 4) void a
     if (wave < nt) f32_put<D>(tile, acc, col, hi);
     __syncthreads();
     f32_combine<D>(smem[0], TL::FLOATS, min(NW, nt), p.scale, bwd_head<float>(p, p.dq, BDQ, bh), q0, S, p.ss[BDQ],
-                   [&](int row) { f32_dq_row<D, CAUSAL>(p, bh, row); });
+                   [&](int row) { f32_dq_row<D, CAUSAL, true>(p, bh, row); });
 }
 
 template <int D, bool CAUSAL>
@@ -247,7 +247,7 @@ __global__ __launch_bounds__(kF32Threads, D >= 128 ? 1 : D >= 64 ? 3 : 4) void a
     asm volatile("" ::: "memory");
     if (t0 + wave < nq) f32_put<D>(tile, dk_acc, col, hi);
     __syncthreads();
-    auto redo = [&](int row) { f32_dkdv_row<D, CAUSAL>(p, bh, row); };
+    auto redo = [&](int row) { f32_dkdv_row<D, CAUSAL, true>(p, bh, row); };
     f32_combine<D>(smem[0], TL::FLOATS, n, p.scale, bwd_head<float>(p, p.dk, BDK, bh), k0, S, p.ss[BDK], redo);
     __syncthreads();
     if (t0 + wave < nq) f32_put<D>(tile, dv_acc, col, hi);

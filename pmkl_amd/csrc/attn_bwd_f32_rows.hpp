@@ -32,25 +32,35 @@ __device__ __forceinline__ float f32_lane(float x, int src) {
 }
 
 // <a, row>: a[d] is held by lane d % 64 in register a[d / 64]; row is this
-// lane's own 16-byte aligned row of D floats.
-template <int D>
+// lane's own 16-byte aligned row of D floats.  LEAN broadcasts a again in every
+// call and 16 elements at a time: kept across the caller's loop, the D values
+// take more scalar registers than a tile kernel has left.  (In the row kernels
+// that costs 15-30%: 1 head of S1 D64, whole call, 10.4 us against 7.6.)
+template <int D, bool LEAN>
 __device__ __forceinline__ float f32_row_dot(const float (&a)[(D + 63) / 64], const float *row) {
     float acc = 0.f;
+    auto four = [&](float x, int h, int d) __attribute__((always_inline)) {
+        const f32x4_t r = *(const f32x4_t *)(row + 64 * h + d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = __builtin_fmaf(f32_lane(x, d + e), r[e], acc);
+    };
 #pragma unroll
     for (int h = 0; h < (D + 63) / 64; ++h) {
         float x = a[h];
-        asm volatile("" : "+v"(x));   // else all D broadcast values are kept across the caller's loop, and spill
+        constexpr int N = D < 64 ? D : 64;
+        if constexpr (LEAN) {
+            asm volatile("" : "+v"(x));
 #pragma unroll 4
-        for (int d = 0; d < (D < 64 ? D : 64); d += 4) {
-            const f32x4_t r = *(const f32x4_t *)(row + 64 * h + d);
+            for (int d = 0; d < N; d += 4) four(x, h, d);
+        } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc = __builtin_fmaf(f32_lane(x, d + e), r[e], acc);
+            for (int d = 0; d < N; d += 4) four(x, h, d);
         }
     }
     return acc;
 }
 
-template <int D, bool CAUSAL>
+template <int D, bool CAUSAL, bool LEAN>
 __device__ __forceinline__ void f32_dq_row(const BwdParams &p, int bh, int qi) {
     constexpr int NE = (D + 63) / 64;   // head_dim elements per lane
     const int lane = threadIdx.x & 63;
@@ -79,8 +89,8 @@ __device__ __forceinline__ void f32_dq_row(const BwdParams &p, int bh, int qi) {
     auto prob = [&](int j0, float &pv, float &dp) __attribute__((always_inline)) {
         const int j = j0 + lane;
         const int jc = j <= last ? j : last;
-        const float s = f32_row_dot<D>(qv, kg + (int64_t)jc * kss);
-        dp = f32_row_dot<D>(dov, vg + (int64_t)jc * vss);
+        const float s = f32_row_dot<D, LEAN>(qv, kg + (int64_t)jc * kss);
+        dp = f32_row_dot<D, LEAN>(dov, vg + (int64_t)jc * vss);
         pv = j <= last ? fast_exp2(__builtin_fmaf(s, c, -lse2)) : 0.f;
     };
 
@@ -131,7 +141,7 @@ __device__ __forceinline__ void f32_dq_row(const BwdParams &p, int bh, int qi) {
     }
 }
 
-template <int D, bool CAUSAL>
+template <int D, bool CAUSAL, bool LEAN>
 __device__ __forceinline__ void f32_dkdv_row(const BwdParams &p, int bh, int kj) {
     constexpr int NE = (D + 63) / 64;
     const int lane = threadIdx.x & 63;
@@ -160,8 +170,8 @@ __device__ __forceinline__ void f32_dkdv_row(const BwdParams &p, int bh, int kj)
     for (int i0 = first; i0 < S; i0 += 64) {
         const int i = i0 + lane;
         const int ic = i < S ? i : S - 1;
-        const float s = f32_row_dot<D>(kv, qg + (int64_t)ic * qss);
-        const float dp = f32_row_dot<D>(vv, dog + (int64_t)ic * doss);
+        const float s = f32_row_dot<D, LEAN>(kv, qg + (int64_t)ic * qss);
+        const float dp = f32_row_dot<D, LEAN>(vv, dog + (int64_t)ic * doss);
         const float pv = i < S ? fast_exp2(__builtin_fmaf(s, c, -lse2g[ic])) : 0.f;
         const float ds = pv * (dp - drowg[ic]);
         const int n = min(64, S - i0);
@@ -190,6 +200,30 @@ __device__ __forceinline__ void f32_dkdv_row(const BwdParams &p, int bh, int kj)
             dv_j[d] = acc_v[e];
         }
     }
+}
+
+constexpr int kF32RowWaves = 4;   // rows per workgroup, one per wave: the B*H*S rows in one sequence
+
+// The query (or key) row of this wave and its head; false past the last.  The
+// dispatch keeps the rows below 2^26.
+__device__ __forceinline__ bool f32_wave_row(const BwdParams &p, int &bh, int &r) {
+    const uint32_t row = blockIdx.x * kF32RowWaves + (threadIdx.x >> 6), S = (uint32_t)p.S;
+    if (row >= (uint32_t)p.BH * S) return false;
+    bh = (int)(row / S);
+    r = (int)(row - (uint32_t)bh * S);
+    return true;
+}
+
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__(kF32RowWaves * 64) void attn_bwd_f32_row_dq_kernel(BwdParams p) {
+    int bh, qi;
+    if (f32_wave_row(p, bh, qi)) f32_dq_row<D, CAUSAL, false>(p, bh, qi);
+}
+
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__(kF32RowWaves * 64) void attn_bwd_f32_row_dkdv_kernel(BwdParams p) {
+    int bh, kj;
+    if (f32_wave_row(p, bh, kj)) f32_dkdv_row<D, CAUSAL, false>(p, bh, kj);
 }
 
 }  // namespace pmkl_amd

@@ -323,7 +323,12 @@ struct BwdKernels {
     int dkdv_threads, dkdv_rows;
     const char *family = "";       // names them for pmkl_attn_bwd_kernel_name: <family>_dq_kernel, <family>_dkdv_kernel
     int ks = -1;                   // template parameter after the mask, -1 if none
+    bool flat = false;             // grid over the B*H*S rows, else (row tile, head)
 };
+// Workgroups of a pass whose workgroups own `rows` rows each.
+int64_t bwd_grid(const BwdKernels &kc, int rows, int64_t BH, int64_t S) {
+    return kc.flat ? (BH * S + rows - 1) / rows : (S + rows - 1) / rows * BH;
+}
 
 template <typename T, int D, int KS>
 BwdKernels pick_bwd(bool causal) {
@@ -348,6 +353,38 @@ BwdKernels pick_bwd_f32(bool causal) {
                 "attn_bwd_f32"};
     return {pmkl_amd::attn_bwd_f32_dq_kernel<D, false>, pmkl_amd::attn_bwd_f32_dkdv_kernel<D, false>, T, R, T, R,
             "attn_bwd_f32"};
+}
+
+template <int D>
+BwdKernels pick_bwd_f32_rows(bool causal) {
+    constexpr int W = pmkl_amd::kF32RowWaves;
+    if (causal)
+        return {pmkl_amd::attn_bwd_f32_row_dq_kernel<D, true>, pmkl_amd::attn_bwd_f32_row_dkdv_kernel<D, true>,
+                64 * W, W, 64 * W, W, "attn_bwd_f32_row", -1, true};
+    return {pmkl_amd::attn_bwd_f32_row_dq_kernel<D, false>, pmkl_amd::attn_bwd_f32_row_dkdv_kernel<D, false>,
+            64 * W, W, 64 * W, W, "attn_bwd_f32_row", -1, true};
+}
+template <int D>
+BwdKernels pick_bwd_f32(bool causal, bool rows) {
+    return rows ? pick_bwd_f32_rows<D>(causal) : pick_bwd_f32<D>(causal);
+}
+
+// fp32 backward a row per wave for short sequences: a 32-row tile costs the same
+// whatever it holds.  Measured tiles / rows, us per backward call (causal, without
+// O):  S 1  8,192 heads D 64 212 / 37, 65,536 heads D 128 6,275 / 761;  S 4  8,192
+// heads D 64 213 / 138;  S 8  128 heads D 64 16.9 / 11.9, D 128 27.7 / 20.0;  S 16
+// 16 heads D 64 17.0 / 13.0;  S 31  16 heads D 128 28.0 / 25.9.  The lines lie
+// where the two meet, by the rows' workgroups (4 rows) per CU: up to S 6 (head_dim
+// 128: 8) rows at any count, then while few of them queue.  A launch's 2^32
+// threads are 2^26 rows here and 2^24 heads there.
+bool bwd_f32_rows(const pmkl_attn_bwd_args *a) {
+    const int64_t S = a->seq_len, D = a->head_dim, rows = a->batch * a->heads * S;
+    if (rows >= (1LL << 26)) return false;
+    if (S <= (D == 128 ? 8 : 6)) return true;
+    const int64_t per_cu = D == 128  ? (S <= 36 ? 1 : 0)
+                           : D == 64 ? (S <= 8 ? 3 : S <= 14 ? 2 : S <= (a->is_causal ? 36 : 28) ? 1 : 0)
+                                     : (S <= 8 ? 2 : S <= 14 ? 1 : 0);
+    return rows <= pmkl_amd::kF32RowWaves * per_cu * cu_count();
 }
 
 // PMKL_ATTN_BWDSPLIT=0: the split form of the 16-bit backward never, =1
@@ -398,9 +435,10 @@ BwdKernels select_bwd(const pmkl_attn_bwd_args *a) {
         if (d == 64) return pick_bwd<_Float16, 64>(causal, split);
         if (d == 128) return pick_bwd<_Float16, 128>(causal, split);
     } else if (dt == PMKL_DTYPE_F32) {
-        if (d == 32) return pick_bwd_f32<32>(causal);
-        if (d == 64) return pick_bwd_f32<64>(causal);
-        if (d == 128) return pick_bwd_f32<128>(causal);
+        const bool rows = bwd_f32_rows(a);
+        if (d == 32) return pick_bwd_f32<32>(causal, rows);
+        if (d == 64) return pick_bwd_f32<64>(causal, rows);
+        if (d == 128) return pick_bwd_f32<128>(causal, rows);
     }
     return {nullptr, nullptr, 0, 0, 0, 0};
 }
@@ -456,8 +494,7 @@ int check_bwd(const pmkl_attn_bwd_args *a, bool *empty) {
     const BwdKernels kc = select_bwd(a);
     PMKL_REQUIRE(kc.dq != nullptr, PMKL_EUNSUPPORTED, "no backward kernel for dtype %d head_dim %lld",
                  (int)a->dtype, (long long)D);
-    const int64_t nq = (S + kc.dq_rows - 1) / kc.dq_rows, nk = (S + kc.dkdv_rows - 1) / kc.dkdv_rows;
-    const int64_t gq = nq * B * H, gk = nk * B * H;
+    const int64_t gq = bwd_grid(kc, kc.dq_rows, B * H, S), gk = bwd_grid(kc, kc.dkdv_rows, B * H, S);
     PMKL_REQUIRE(std::max(gq, gk) <= 0x7fffffffLL, PMKL_EINVAL, "grid too large (%lld workgroups)",
                  (long long)std::max(gq, gk));
     return PMKL_OK;
@@ -471,7 +508,7 @@ int launch_bwd(const pmkl_attn_bwd_args *a, float *ws, void *stream) {
     const int64_t B = a->batch, H = a->heads, S = a->seq_len, D = a->head_dim;
     const BwdKernels kc = select_bwd(a);
     const int64_t nq = (S + kc.dq_rows - 1) / kc.dq_rows, nk = (S + kc.dkdv_rows - 1) / kc.dkdv_rows;
-    const int64_t gq = nq * B * H, gk = nk * B * H;
+    const int64_t gq = bwd_grid(kc, kc.dq_rows, B * H, S), gk = bwd_grid(kc, kc.dkdv_rows, B * H, S);
 
     BwdParams p;
     p.q = a->q;
@@ -738,8 +775,8 @@ const char *pmkl_attn_bwd_kernel_name(const pmkl_attn_bwd_args *a) {
     snprintf(args, sizeof(args), "<%s%lld, %s%s>", dt, (long long)a->head_dim, a->is_causal ? "causal" : "full", ks);
     const int64_t BH = a->batch * a->heads;
     snprintf(name, sizeof(name), "%s_dq_kernel%s grid %lld x %d, %s_dkdv_kernel%s grid %lld x %d", kc.family, args,
-             (long long)((a->seq_len + kc.dq_rows - 1) / kc.dq_rows * BH), kc.dq_threads, kc.family, args,
-             (long long)((a->seq_len + kc.dkdv_rows - 1) / kc.dkdv_rows * BH), kc.dkdv_threads);
+             (long long)bwd_grid(kc, kc.dq_rows, BH, a->seq_len), kc.dq_threads, kc.family, args,
+             (long long)bwd_grid(kc, kc.dkdv_rows, BH, a->seq_len), kc.dkdv_threads);
     return name;
 }
 
