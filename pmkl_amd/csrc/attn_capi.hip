@@ -314,6 +314,14 @@ int check_no_self_overlap(const char *name, const int64_t st[3], int64_t B, int6
     return PMKL_OK;
 }
 
+// A launch's grid is counted in threads, in 32 bits; HIP cuts what passes them
+// off without an error.
+int check_grid(int64_t workgroups, int threads) {
+    PMKL_REQUIRE(workgroups <= 0x7fffffffLL && workgroups * threads < (1LL << 32), PMKL_EINVAL,
+                 "grid too large (%lld workgroups)", (long long)workgroups);
+    return PMKL_OK;
+}
+
 using pmkl_amd::BwdParams;
 typedef void (*bwd_kernel_fn)(BwdParams);
 
@@ -494,10 +502,8 @@ int check_bwd(const pmkl_attn_bwd_args *a, bool *empty) {
     const BwdKernels kc = select_bwd(a);
     PMKL_REQUIRE(kc.dq != nullptr, PMKL_EUNSUPPORTED, "no backward kernel for dtype %d head_dim %lld",
                  (int)a->dtype, (long long)D);
-    const int64_t gq = bwd_grid(kc, kc.dq_rows, B * H, S), gk = bwd_grid(kc, kc.dkdv_rows, B * H, S);
-    PMKL_REQUIRE(std::max(gq, gk) <= 0x7fffffffLL, PMKL_EINVAL, "grid too large (%lld workgroups)",
-                 (long long)std::max(gq, gk));
-    return PMKL_OK;
+    if ((rc = check_grid(bwd_grid(kc, kc.dq_rows, B * H, S), kc.dq_threads)) != PMKL_OK) return rc;
+    return check_grid(bwd_grid(kc, kc.dkdv_rows, B * H, S), kc.dkdv_threads);
 }
 
 // Launches the two backward passes of a validated, non-empty call.  ws holds
@@ -715,6 +721,7 @@ int plan_fwd(const pmkl_attn_fwd_args *a, FwdPlan *pl) {
         PMKL_REQUIRE(cus > 0, PMKL_EHIP, "could not read the device's CU count");
         grid = std::min<int64_t>(grid, (int64_t)kc.per_cu * cus);
     }
+    if ((rc = check_grid(grid, kc.threads)) != PMKL_OK) return rc;
     pl->kc = kc;
     pl->grid = grid;
     return PMKL_OK;

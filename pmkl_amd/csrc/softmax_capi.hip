@@ -133,6 +133,9 @@ int pmkl_softmax_fwd(const pmkl_softmax_args *a, void *stream) {
     p.log2g = g;
     const int64_t rows_per_block = int64_t(pmkl_amd::kSoftmaxThreads / 64) << (6 - g);
     const int64_t blocks = (a->batch + rows_per_block - 1) / rows_per_block;
+    // a launch's grid is counted in threads, in 32 bits
+    PMKL_REQUIRE(blocks * pmkl_amd::kSoftmaxThreads < (int64_t(1) << 32), PMKL_EINVAL, "grid too large (%lld workgroups)",
+                 (long long)blocks);
     hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(pmkl_amd::kSoftmaxThreads), 0, (hipStream_t)stream, p);
     const hipError_t err = hipGetLastError();
     PMKL_REQUIRE(err == hipSuccess, PMKL_EHIP, "softmax launch failed: %s", hipGetErrorString(err));

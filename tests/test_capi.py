@@ -330,3 +330,19 @@ def test_backward_kernel_name_query():
                       "attn_bwd_dkdv_kernel<bf16, 64, causal, 1> grid 6 x 256")
     assert name(dtype=capi.PMKL_DTYPE_F32, D=128, causal=False) == (
         "attn_bwd_f32_dq_kernel<128, full> grid 20 x 256, attn_bwd_f32_dkdv_kernel<128, full> grid 20 x 256")
+
+
+def test_launches_past_2_32_threads_are_refused():
+    """HIP cuts the grid of such a launch off without an error."""
+    f32 = dict(dtype=capi.PMKL_DTYPE_F32, ml_dtype=capi.PMKL_DTYPE_F32)
+    for BH, S, kw in ((1 << 23, 200, {}), (1 << 24, 128, f32)):
+        assert capi.attn_fwd_kernel_name(_args(batch=BH, heads=1, seq_len=S, **kw)) is None
+        assert "grid too large" in capi.last_error()
+        assert capi.attn_fwd_kernel_name(_args(batch=BH - 1, heads=1, seq_len=S, **kw)) is not None, capi.last_error()
+    bwd = lambda BH, S, dtype: capi.attn_bwd_kernel_name(capi.make_bwd_args(
+        *(range(0x1000, 0xb000, 0x1000)), 0, 0, dtype=dtype, batch=BH, heads=1, seq_len=S, head_dim=64))
+    for BH, S, dtype in ((1 << 24, 128, capi.PMKL_DTYPE_BF16), (1 << 24, 8, capi.PMKL_DTYPE_F32)):
+        assert bwd(BH, S, dtype) is None and "grid too large" in capi.last_error()
+        assert bwd(BH - 1, S, dtype) is not None, capi.last_error()
+    a = capi.make_softmax_args(0x1000, 0x1000, out_dtype=0, in_dtype=0, elements=40, stride=40, batch=1 << 28)
+    assert capi.softmax_raw(a) == capi.PMKL_EINVAL and "grid too large" in capi.last_error()
