@@ -406,13 +406,17 @@ int bwd_split_mode() {
 }
 // Split form of the 16-bit backward (attn_bwd_kernels.hpp, KS = 2): where the
 // 128-row workgroups leave CUs idle, or are so few that the longest causal one
-// sets the time.  It costs a quarter more once they fill the chip.  Measured
+// sets the time.  It costs a quarter more once they fill the chip, and a tenth on
+// a single tile of streamed rows, where there is nothing to split (so from S 65 on;
+// at head_dim 64 and 128 full, where the second tile costs a whole one, from S 80).  Measured
 // without / with it, us per backward call (bf16, without O), by 128-row workgroups:
-//   head_dim 128 full    128: 152.9 / 117.0 (S 2047), 36.7 / 29.7 (S 200);  256: 174 / 218, 38.9 / 55.2
+//   head_dim 128 S 64    1: 16.5 / 18.7
+//                full    128: 152.9 / 117.0 (S 2047), 36.7 / 29.7 (S 200);  256: 174 / 218, 38.9 / 55.2
 //                causal  128: 156.9 / 107.2;  256: 158 / 131 (S 2047), 90.1 / 83.6 (S 1024), 57.7 / 61.7 (S 512);
 //                        512: 196 / 252
 //   head_dim 64  full    128: 99.3 / 70.4;  256: 105.7 / 105.0 (S 2047), 24.0 / 25.5 (S 200)
 //                causal  256: 104.3 / 79.7 (S 2047), 23.9 / 22.2 (S 200);  512: 122 / 121 (S 2047), 46.1 / 54.1 (S 512)
+//                        192: 24.6 / 23.3, 255: 25.0 / 26.1 (S 320); with O, S 100: 128 1.12 times faster, 192 0.92
 //   head_dim 32  full    256: 75.4 / 65.5 (S 2047), 23.3 / 21.6 (S 200);  512: 112 / 121
 //                causal  256: 78.9 / 53.7;  512: 82.6 / 72.8 (S 2047), 47.1 / 42.9 (S 1024);  1,024: 121 / 132
 bool bwd_split(const pmkl_attn_bwd_args *a) {
@@ -420,11 +424,13 @@ bool bwd_split(const pmkl_attn_bwd_args *a) {
     // its dK/dV pass addresses 128 rows of Q and dout by one 32-bit buffer range
     if (std::max(a->q_strides[2], a->dout_strides[2]) * 2 * 128 >= (1LL << 31)) return false;
     if (bwd_split_mode() >= 0) return bwd_split_mode() == 1;
-    const bool long_causal = a->is_causal != 0 && S >= 1024;
+    const bool causal = a->is_causal != 0, long_causal = causal && S >= 1024;
+    if (S <= 64 || (!causal && D >= 64 && S < 80)) return false;
     const int64_t cus = cu_count(), groups = a->batch * a->heads * ((S + 127) / 128);
-    const int64_t most = D == 128  ? (long_causal ? cus : cus / 2)
-                         : D == 64 ? (a->is_causal != 0 ? cus : cus / 2)
-                                   : (long_causal ? 2 * cus : cus);
+    // causal head_dim 64: an odd 64-row tile runs beside others in the 128-row form
+    const int64_t tiles = (S + 63) / 64;
+    const int64_t most64 = !causal || tiles <= 2 ? cus / 2 : tiles == 3 || tiles == 5 ? 3 * cus / 4 : cus;
+    const int64_t most = D == 128 ? (long_causal ? cus : cus / 2) : D == 64 ? most64 : (long_causal ? 2 * cus : cus);
     return groups <= most;
 }
 

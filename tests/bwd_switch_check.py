@@ -34,8 +34,8 @@ def main() -> int:
         for D in (32, 64, 128):
             for causal in (True, False):
                 t.test_bwd_small_shapes_vs_oracle(dev, dtype, D, causal)
-                # odd and even counts of 64-row tiles, more than two per workgroup
-                for B, H, S in ((1, 1, 321), (1, 2, 449), (1, 1, 700)):
+                # edges of a wave's rows and of a tile, odd and even counts of tiles, more than two per workgroup
+                for B, H, S in ((1, 3, 31), (1, 2, 127), (1, 2, 129), (1, 1, 193), (1, 1, 321), (1, 2, 449), (1, 1, 700)):
                     tag = f"{dtype} B{B} H{H} S{S} D{D} causal={causal}"
                     t._say(f"case {tag}")
                     got, ref, _ = t._run(B, H, S, D, dtype, causal, seed=9500 + S, ml_dtype=torch.float32)

@@ -16,6 +16,27 @@ pytestmark = pytest.mark.gpu
 ROOT = Path(__file__).resolve().parent.parent
 
 
+def test_backward_form_rule(device):
+    """The split form where it is the faster (bf16, 256 CUs): not on a single tile
+    of streamed rows, not where the 128-row workgroups fill the CUs."""
+    from pmkl_amd import capi
+
+    def ks(BH, S, D, causal):
+        name = capi.attn_bwd_kernel_name(capi.make_bwd_args(
+            *(range(0x1000, 0xb000, 0x1000)), 0, 0, dtype=capi.PMKL_DTYPE_BF16, batch=1, heads=BH, seq_len=S, head_dim=D,
+            is_causal=causal))
+        return int(name.split(">")[0].split(", ")[3])
+
+    for BH, S, D, causal in ((1, 65, 128, True), (128, 100, 64, True), (96, 129, 64, True), (64, 320, 64, True),
+                             (128, 256, 64, True), (64, 512, 64, True), (1, 80, 64, False), (128, 128, 128, False),
+                             (16, 2047, 128, True), (256, 128, 32, False), (32, 2047, 32, True)):
+        assert ks(BH, S, D, causal) == 2, (BH, S, D, causal)
+    for BH, S, D, causal in ((1, 1, 128, True), (1, 64, 128, True), (4, 33, 64, False), (16, 64, 32, True),
+                             (192, 100, 64, True), (128, 129, 64, True), (85, 320, 64, True), (1, 65, 64, False),
+                             (192, 128, 128, False), (64, 512, 128, True), (72, 512, 64, True), (300, 128, 32, False)):
+        assert ks(BH, S, D, causal) == 1, (BH, S, D, causal)
+
+
 @pytest.mark.parametrize("split", ["0", "1"])
 def test_backward_form_vs_oracle(device, split):
     env = {k: v for k, v in os.environ.items() if not k.startswith("PMKL_ATTN")}

@@ -1,7 +1,8 @@
-"""The 16-bit backward's split form (two waves per 32 owned rows) at the sizes
-where it can go wrong: one row, the edges of a wave's rows, of a workgroup's 64
-and of the 64 and 128 streamed rows, an odd number of tiles; and the 128-row
-form beside it on grids too large for the split.  Against the float64 oracle
+"""The 16-bit backward in the form that the dispatch chooses, with and without
+the forward's output: the split form (two waves per 32 owned rows) from S 65 on
+at the edges of a wave's rows, of a workgroup's 64 and of the 64 and 128
+streamed rows and an odd number of tiles; the 128-row form below and on grids
+too large for the split (test_bwd_forms_gpu.py pins either at all sizes).  Against the float64 oracle
 with the tolerances of the other backward tests; with the forward's output
 against the same oracle with its row term moved to <dout, O> (_move_row_term)."""
 from __future__ import annotations
