@@ -178,7 +178,7 @@ int pmkl_attn_bwd_supported(int32_t dtype, int64_t head_dim);
 
 /* The two kernels pmkl_attn_bwd would launch for these arguments (the workspace
  * is not looked at), with their launch shapes, e.g.
- * "attn_bwd_dq_kernel<bf16, 64, causal, 2> grid 32 x 256, attn_bwd_dkdv_kernel<bf16, 64, causal, 2> grid 32 x 256";
+ * "attn_bwd_dq_kernel<bf16, 64, causal, 2, 4> grid 32 x 256, attn_bwd_dkdv_kernel<bf16, 64, causal, 2, 4> grid 32 x 256";
  * otherwise as pmkl_attn_fwd_kernel_name, with a string of its own.  An addition
  * to ABI version 5. */
 const char *pmkl_attn_bwd_kernel_name(const pmkl_attn_bwd_args *args);

@@ -67,13 +67,12 @@ __device__ __forceinline__ T *bwd_head(const BwdParams &p, const void *base, int
     return (T *)base + (int64_t)b * p.sb[t] + (int64_t)h * p.sh[t];
 }
 
-// Waves per workgroup (32 / KS owned rows each): one per SIMD, with up to 512 registers at head_dim 128
-// (the pipelined dQ loop's two score sets, the dK/dV accumulators), 256 below,
-// where two workgroups share a CU.  (One workgroup of eight waves instead runs
-// all their phases in step: B64 H8 S256 D32 19.4 / 22.0 us against 16.8 / 17.4.)
-template <int D> constexpr int bwd_waves_dq() { return 4; }
-template <int D> constexpr int bwd_waves_dkdv() { return 4; }
-
+// NW waves per workgroup (32 / KS owned rows each).  Four, one per SIMD, with up
+// to 512 registers at head_dim 128 (the pipelined dQ loop's two score sets, the
+// dK/dV accumulators), 256 below, where two workgroups share a CU.  Eight at
+// head_dim 64 stage every streamed tile once for 256 rows, but run all their
+// phases in step and come in twice as large pieces (attn_capi.hip has the rule;
+// B64 H8 S256 D32 19.4 / 22.0 us a pass with eight, 16.8 / 17.4 with four).
 // 16-byte chunk (logical chunk pc of row `row`) staging of a 64-row tile:
 // loads go to registers ahead of use (the dK/dV pass one tile ahead, the
 // dQ pass's plain loop below head_dim 128), LDS writes place the chunk at its
@@ -87,8 +86,8 @@ struct BwdTile {
     static constexpr int BN = BN_;              // streamed rows per tile
     static constexpr int CPR = D / 8;
     static constexpr int CHUNKS = BN * CPR;
-    static constexpr int LOADS = (CHUNKS + THREADS - 1) / THREADS;
-    static constexpr bool PARTIAL = CHUNKS % THREADS != 0;
+    static constexpr int LOADS = CHUNKS / THREADS;
+    static_assert(CHUNKS % THREADS == 0, "a tile splits evenly over the threads");
 };
 
 // Buffer resource of the rows [r0, S) of a [S, D] matrix with row stride ss
@@ -164,14 +163,13 @@ __device__ __forceinline__ void bwd_lds_dma16(__amdgpu_buffer_rsrc_t r, int off,
 // ---------------------------------------------------------------------------
 // pass 1: dQ (and the row vectors D_n, log2-sum-exp)
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool CAUSAL, int KS = 1>
-__global__ __launch_bounds__(bwd_waves_dq<D>() * 64, D >= 128 ? 1 : 2) void attn_bwd_dq_kernel(BwdParams p) {
+template <typename T, int D, bool CAUSAL, int KS = 1, int NW = 4>
+__global__ __launch_bounds__(NW * 64, D >= 128 ? 1 : 2) void attn_bwd_dq_kernel(BwdParams p) {
     using E = Elt16<T>;
     using frag = typename E::frag;
-    using TL = BwdTile<T, D, bwd_waves_dq<D>(), KS>;
+    using TL = BwdTile<T, D, NW, KS>;
     constexpr int BN = TL::BN, CPR = TL::CPR, LOADS = TL::LOADS;
     constexpr int kBwdThreads = TL::THREADS, kBwdRows = TL::ROWS;
-    constexpr bool PARTIAL = TL::PARTIAL;
     constexpr int NDB = D / 32, NDK = D / 16;
     constexpr int NKB = 2 / KS;   // 32-key blocks of a tile per wave
 
@@ -238,7 +236,6 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, D >= 128 ? 1 : 2) void attn
     const unsigned lds_w = (unsigned)(uintptr_t)(__attribute__((address_space(3))) T *)&smem[0][0][0] + 1024u * wave;
     // All DMAs of tile kt into stage kt % 3 (rows past S read as zero).
     auto dma_tile = [&](int kt) __attribute__((always_inline)) {
-        static_assert(!PIPE || !PARTIAL, "the DMA staging covers whole tiles");
         const auto kr = bwd_rows_rsrc<T, D>(kg, kt * BN, S, kss);
         const auto vr = bwd_rows_rsrc<T, D>(vg, kt * BN, S, vss);
         const unsigned base = lds_w + (unsigned)((kt % 3) * 2 * TILE_BYTES);
@@ -269,22 +266,19 @@ __global__ __launch_bounds__(bwd_waves_dq<D>() * 64, D >= 128 ? 1 : 2) void attn
         const auto kr = bwd_rows_rsrc<T, D>(kg, kt * BN, S, kss);
         const auto vr = bwd_rows_rsrc<T, D>(vg, kt * BN, S, vss);
 #pragma unroll
-        for (int j = 0; j < LOADS; ++j)
-            if (!PARTIAL || j * kBwdThreads + tid < TL::CHUNKS) {
-                kreg2[SET][j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(kr, goffk[j], 0, 0));
-                vreg2[SET][j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(vr, goffv[j], 0, 0));
-            }
+        for (int j = 0; j < LOADS; ++j) {
+            kreg2[SET][j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(kr, goffk[j], 0, 0));
+            vreg2[SET][j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(vr, goffv[j], 0, 0));
+        }
     };
     auto swrite2 = [&](int st, auto set_c) __attribute__((always_inline)) {
         constexpr int SET = decltype(set_c)::value;
 #pragma unroll
         for (int j = 0; j < LOADS; ++j) {
             const int sl = j * kBwdThreads + tid;
-            if (!PARTIAL || sl < TL::CHUNKS) {
-                const int row = sl / CPR, pc = sl % CPR;
-                *(u32x4_t *)(&smem[st][0][row * D + 8 * (pc ^ swz_b<CPR>(row))]) = kreg2[SET][j];
-                *(u32x4_t *)(&smem[st][1][row * D + 8 * (pc ^ swz_b<CPR>(row))]) = vreg2[SET][j];
-            }
+            const int row = sl / CPR, pc = sl % CPR;
+            *(u32x4_t *)(&smem[st][0][row * D + 8 * (pc ^ swz_b<CPR>(row))]) = kreg2[SET][j];
+            *(u32x4_t *)(&smem[st][1][row * D + 8 * (pc ^ swz_b<CPR>(row))]) = vreg2[SET][j];
         }
     };
 
@@ -585,14 +579,13 @@ __device__ __forceinline__ int bwd_dkdv_mlim(int qbase, int k0w, int kj, int hi)
     return CAUSAL && qbase < k0w + 31 ? kj - qbase - 16 * hi : -64;
 }
 
-template <typename T, int D, bool CAUSAL, int KS = 1>
-__global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, D >= 128 ? 1 : 2) void attn_bwd_dkdv_kernel(BwdParams p) {
+template <typename T, int D, bool CAUSAL, int KS = 1, int NW = 4>
+__global__ __launch_bounds__(NW * 64, D >= 128 ? 1 : 2) void attn_bwd_dkdv_kernel(BwdParams p) {
     using E = Elt16<T>;
     using frag = typename E::frag;
-    using TL = BwdTile<T, D, bwd_waves_dkdv<D>(), KS, 64 * KS>;
+    using TL = BwdTile<T, D, NW, KS, 64 * KS>;
     constexpr int BN = TL::BN, CPR = TL::CPR, LOADS = TL::LOADS;
     constexpr int kBwdThreads = TL::THREADS, kBwdRows = TL::ROWS;
-    constexpr bool PARTIAL = TL::PARTIAL;
     constexpr int NDB = D / 32, NDK = D / 16;
 
     // [stage][Q, dout]; row vectors [stage][lse2, D_n]
@@ -652,11 +645,10 @@ __global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, D >= 128 ? 1 : 2) void at
         const auto qr = bwd_rows_rsrc<T, D, BN>(qg, qtl * BN, S, qss);
         const auto orr = bwd_rows_rsrc<T, D, BN>(dog, qtl * BN, S, doss);
 #pragma unroll
-        for (int j = 0; j < LOADS; ++j)
-            if (!PARTIAL || j * kBwdThreads + tid < TL::CHUNKS) {
-                qreg[j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(qr, goffq[j], 0, 0));
-                oreg[j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(orr, goffo[j], 0, 0));
-            }
+        for (int j = 0; j < LOADS; ++j) {
+            qreg[j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(qr, goffq[j], 0, 0));
+            oreg[j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(orr, goffo[j], 0, 0));
+        }
         if (tid < 2 * BN) {
             const int row = qtl * BN + (tid & (BN - 1));
             // rows past S: lse2 = +inf gives P = 0 (their scores are masked too)
@@ -667,11 +659,9 @@ __global__ __launch_bounds__(bwd_waves_dkdv<D>() * 64, D >= 128 ? 1 : 2) void at
 #pragma unroll
         for (int j = 0; j < LOADS; ++j) {
             const int sl = j * kBwdThreads + tid;
-            if (!PARTIAL || sl < TL::CHUNKS) {
-                const int row = sl / CPR, pc = sl % CPR;
-                *(u32x4_t *)(&smem[st][0][row * D + 8 * (pc ^ swz_b<CPR>(row))]) = qreg[j];
-                *(u32x4_t *)(&smem[st][1][row * D + 8 * (pc ^ swz_b<CPR>(row))]) = oreg[j];
-            }
+            const int row = sl / CPR, pc = sl % CPR;
+            *(u32x4_t *)(&smem[st][0][row * D + 8 * (pc ^ swz_b<CPR>(row))]) = qreg[j];
+            *(u32x4_t *)(&smem[st][1][row * D + 8 * (pc ^ swz_b<CPR>(row))]) = oreg[j];
         }
         if (tid < 2 * BN) svec[st][tid / BN][tid & (BN - 1)] = vreg;
     };

@@ -1,4 +1,4 @@
-// Explicit instantiations of the key-split 16-bit backward for _Float16: compiled as
+// Explicit instantiations of the key-split and the eight-wave 16-bit backward for _Float16: compiled as
 // a translation unit of its own so that the library's kernels build in parallel
 // (attn_capi.hip declares them extern).
 #include <hip/hip_runtime.h>
@@ -18,4 +18,8 @@ template __global__ void attn_bwd_dq_kernel<_Float16, 128, true, 2>(BwdParams);
 template __global__ void attn_bwd_dq_kernel<_Float16, 128, false, 2>(BwdParams);
 template __global__ void attn_bwd_dkdv_kernel<_Float16, 128, true, 2>(BwdParams);
 template __global__ void attn_bwd_dkdv_kernel<_Float16, 128, false, 2>(BwdParams);
+template __global__ void attn_bwd_dq_kernel<_Float16, 64, true, 1, 8>(BwdParams);
+template __global__ void attn_bwd_dq_kernel<_Float16, 64, false, 1, 8>(BwdParams);
+template __global__ void attn_bwd_dkdv_kernel<_Float16, 64, true, 1, 8>(BwdParams);
+template __global__ void attn_bwd_dkdv_kernel<_Float16, 64, false, 1, 8>(BwdParams);
 }  // namespace pmkl_amd

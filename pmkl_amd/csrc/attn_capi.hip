@@ -47,7 +47,7 @@ extern template __global__ void attn_fwd_w64_kernel<__bf16, 128, true, 1, 4>(Att
 extern template __global__ void attn_fwd_w64_kernel<_Float16, 128, true, 1, 4>(AttnParams);
 extern template __global__ void attn_fwd_w64_kernel<__bf16, 128, false, 1, 4>(AttnParams);
 extern template __global__ void attn_fwd_w64_kernel<_Float16, 128, false, 1, 4>(AttnParams);
-// The key-split form of the 16-bit backward: attn_bwd_split_<dtype>.hip.
+// The key-split and the eight-wave forms of the 16-bit backward: attn_bwd_split_<dtype>.hip.
 #define PMKL_BWD_SPLIT_EXTERN(T, D)                                                    \
     extern template __global__ void attn_bwd_dq_kernel<T, D, true, 2>(BwdParams);      \
     extern template __global__ void attn_bwd_dq_kernel<T, D, false, 2>(BwdParams);     \
@@ -60,6 +60,14 @@ PMKL_BWD_SPLIT_EXTERN(_Float16, 32)
 PMKL_BWD_SPLIT_EXTERN(_Float16, 64)
 PMKL_BWD_SPLIT_EXTERN(_Float16, 128)
 #undef PMKL_BWD_SPLIT_EXTERN
+#define PMKL_BWD_EIGHT_EXTERN(T)                                                         \
+    extern template __global__ void attn_bwd_dq_kernel<T, 64, true, 1, 8>(BwdParams);    \
+    extern template __global__ void attn_bwd_dq_kernel<T, 64, false, 1, 8>(BwdParams);   \
+    extern template __global__ void attn_bwd_dkdv_kernel<T, 64, true, 1, 8>(BwdParams);  \
+    extern template __global__ void attn_bwd_dkdv_kernel<T, 64, false, 1, 8>(BwdParams);
+PMKL_BWD_EIGHT_EXTERN(__bf16)
+PMKL_BWD_EIGHT_EXTERN(_Float16)
+#undef PMKL_BWD_EIGHT_EXTERN
 }  // namespace pmkl_amd
 
 namespace {
@@ -330,7 +338,7 @@ struct BwdKernels {
     int dq_threads, dq_rows;       // threads and owned rows per workgroup
     int dkdv_threads, dkdv_rows;
     const char *family = "";       // names them for pmkl_attn_bwd_kernel_name: <family>_dq_kernel, <family>_dkdv_kernel
-    int ks = -1;                   // template parameter after the mask, -1 if none
+    int ks = -1, nw = -1;          // template parameters after the mask, -1 if none
     bool flat = false;             // grid over the B*H*S rows, else (row tile, head)
 };
 // Workgroups of a pass whose workgroups own `rows` rows each.
@@ -338,19 +346,20 @@ int64_t bwd_grid(const BwdKernels &kc, int rows, int64_t BH, int64_t S) {
     return kc.flat ? (BH * S + rows - 1) / rows : (S + rows - 1) / rows * BH;
 }
 
-template <typename T, int D, int KS>
+template <typename T, int D, int KS, int NW>
 BwdKernels pick_bwd(bool causal) {
-    using TQ = pmkl_amd::BwdTile<T, D, pmkl_amd::bwd_waves_dq<D>(), KS>;
-    using TK = pmkl_amd::BwdTile<T, D, pmkl_amd::bwd_waves_dkdv<D>(), KS>;
+    using TL = pmkl_amd::BwdTile<T, D, NW, KS>;
     if (causal)
-        return {pmkl_amd::attn_bwd_dq_kernel<T, D, true, KS>, pmkl_amd::attn_bwd_dkdv_kernel<T, D, true, KS>,
-                TQ::THREADS, TQ::ROWS, TK::THREADS, TK::ROWS, "attn_bwd", KS};
-    return {pmkl_amd::attn_bwd_dq_kernel<T, D, false, KS>, pmkl_amd::attn_bwd_dkdv_kernel<T, D, false, KS>,
-            TQ::THREADS, TQ::ROWS, TK::THREADS, TK::ROWS, "attn_bwd", KS};
+        return {pmkl_amd::attn_bwd_dq_kernel<T, D, true, KS, NW>, pmkl_amd::attn_bwd_dkdv_kernel<T, D, true, KS, NW>,
+                TL::THREADS, TL::ROWS, TL::THREADS, TL::ROWS, "attn_bwd", KS, NW};
+    return {pmkl_amd::attn_bwd_dq_kernel<T, D, false, KS, NW>, pmkl_amd::attn_bwd_dkdv_kernel<T, D, false, KS, NW>,
+            TL::THREADS, TL::ROWS, TL::THREADS, TL::ROWS, "attn_bwd", KS, NW};
 }
 template <typename T, int D>
-BwdKernels pick_bwd(bool causal, bool split) {
-    return split ? pick_bwd<T, D, 2>(causal) : pick_bwd<T, D, 1>(causal);
+BwdKernels pick_bwd(bool causal, bool split, bool eight) {
+    if constexpr (D == 64)
+        if (eight) return pick_bwd<T, D, 1, 8>(causal);
+    return split ? pick_bwd<T, D, 2, 4>(causal) : pick_bwd<T, D, 1, 4>(causal);
 }
 
 template <int D>
@@ -368,9 +377,9 @@ BwdKernels pick_bwd_f32_rows(bool causal) {
     constexpr int W = pmkl_amd::kF32RowWaves;
     if (causal)
         return {pmkl_amd::attn_bwd_f32_row_dq_kernel<D, true>, pmkl_amd::attn_bwd_f32_row_dkdv_kernel<D, true>,
-                64 * W, W, 64 * W, W, "attn_bwd_f32_row", -1, true};
+                64 * W, W, 64 * W, W, "attn_bwd_f32_row", -1, -1, true};
     return {pmkl_amd::attn_bwd_f32_row_dq_kernel<D, false>, pmkl_amd::attn_bwd_f32_row_dkdv_kernel<D, false>,
-            64 * W, W, 64 * W, W, "attn_bwd_f32_row", -1, true};
+            64 * W, W, 64 * W, W, "attn_bwd_f32_row", -1, -1, true};
 }
 template <int D>
 BwdKernels pick_bwd_f32(bool causal, bool rows) {
@@ -410,7 +419,7 @@ int bwd_split_mode() {
 // a single tile of streamed rows, where there is nothing to split (so from S 65 on;
 // at head_dim 64 and 128 full, where the second tile costs a whole one, from S 80).  Measured
 // without / with it, us per backward call (bf16, without O), by 128-row workgroups:
-//   head_dim 128 S 64    1: 16.5 / 18.7
+//   head_dim 128 S 64    1: 16.3 / 18.7
 //                full    128: 152.9 / 117.0 (S 2047), 36.7 / 29.7 (S 200);  256: 174 / 218, 38.9 / 55.2
 //                causal  128: 156.9 / 107.2;  256: 158 / 131 (S 2047), 90.1 / 83.6 (S 1024), 57.7 / 61.7 (S 512);
 //                        512: 196 / 252
@@ -434,20 +443,50 @@ bool bwd_split(const pmkl_attn_bwd_args *a) {
     return groups <= most;
 }
 
+// PMKL_ATTN_BWDWAVES=4 or 8 pins the waves of the 128-row form at head_dim 64; 0 if unset (read once).
+int bwd_waves_mode() {
+    static const int v = [] {
+        const char *e = getenv("PMKL_ATTN_BWDWAVES");
+        return e ? (atoi(e) == 8 ? 8 : 4) : 0;
+    }();
+    return v;
+}
+// Eight waves (256-row workgroups, one per CU) at head_dim 64 on long sequences:
+// they stage each streamed tile once where two four-wave workgroups do so twice,
+// but a CU takes 256 rows or none, so only where every CU's share of 128-row
+// workgroups is an even number.  Measured with four / eight waves, us per backward
+// call (bf16, with O), by 128-row workgroups:
+//   full    S 2048  384: 120.0 / 111.5, 768: 196.6 / 233.3;  S 8192  384: 440 / 397, 512: 487 / 464, 896: 921 / 857,
+//           1024: 953 / 926, 1280: 1,190 / 1,309, 1536: 1,414 / 1,378;  S 1024  288: 65.5 / 63.0, 512: 75.3 / 81.6
+//           (without O  320: 78.7 / 82.4)
+//   causal  S 8192  1024: 542 / 504, 768: 411 / 447, 512: 335 / 411;  S 2048  1024: 154.5 / 151.8, 640: 104 / 118
+bool bwd_eight(const pmkl_attn_bwd_args *a, bool split) {
+    const int64_t S = a->seq_len, cus = cu_count();
+    if (split || a->head_dim != 64) return false;
+    if (bwd_waves_mode() != 0) return bwd_waves_mode() == 8;
+    if (cus <= 0 || S < 768) return false;
+    const int64_t groups = a->batch * a->heads * ((S + 127) / 128), share = (groups + cus - 1) / cus;
+    if (a->is_causal != 0) return S >= 4096 && share == 4;
+    if (S < 1536) return share == 2 && a->o != nullptr && groups <= 7 * cus / 4;
+    return share == 2 || (S >= 4096 && (share == 4 || share == 6));
+}
+
 BwdKernels select_bwd(const pmkl_attn_bwd_args *a) {
     const int32_t dt = a->dtype;
     const int64_t d = a->head_dim;
     const bool causal = a->is_causal != 0;
     if (dt == PMKL_DTYPE_BF16) {
         const bool split = bwd_split(a);
-        if (d == 32) return pick_bwd<__bf16, 32>(causal, split);
-        if (d == 64) return pick_bwd<__bf16, 64>(causal, split);
-        if (d == 128) return pick_bwd<__bf16, 128>(causal, split);
+        const bool eight = bwd_eight(a, split);
+        if (d == 32) return pick_bwd<__bf16, 32>(causal, split, eight);
+        if (d == 64) return pick_bwd<__bf16, 64>(causal, split, eight);
+        if (d == 128) return pick_bwd<__bf16, 128>(causal, split, eight);
     } else if (dt == PMKL_DTYPE_F16) {
         const bool split = bwd_split(a);
-        if (d == 32) return pick_bwd<_Float16, 32>(causal, split);
-        if (d == 64) return pick_bwd<_Float16, 64>(causal, split);
-        if (d == 128) return pick_bwd<_Float16, 128>(causal, split);
+        const bool eight = bwd_eight(a, split);
+        if (d == 32) return pick_bwd<_Float16, 32>(causal, split, eight);
+        if (d == 64) return pick_bwd<_Float16, 64>(causal, split, eight);
+        if (d == 128) return pick_bwd<_Float16, 128>(causal, split, eight);
     } else if (dt == PMKL_DTYPE_F32) {
         const bool rows = bwd_f32_rows(a);
         if (d == 32) return pick_bwd_f32<32>(causal, rows);
@@ -783,8 +822,8 @@ const char *pmkl_attn_bwd_kernel_name(const pmkl_attn_bwd_args *a) {
     if (empty) return "none";
     const BwdKernels kc = select_bwd(a);
     const char *dt = a->dtype == PMKL_DTYPE_BF16 ? "bf16, " : a->dtype == PMKL_DTYPE_F16 ? "fp16, " : "";
-    char args[64], ks[16] = "";
-    if (kc.ks >= 0) snprintf(ks, sizeof(ks), ", %d", kc.ks);
+    char args[64], ks[24] = "";
+    if (kc.ks >= 0) snprintf(ks, sizeof(ks), ", %d, %d", kc.ks, kc.nw);
     snprintf(args, sizeof(args), "<%s%lld, %s%s>", dt, (long long)a->head_dim, a->is_causal ? "causal" : "full", ks);
     const int64_t BH = a->batch * a->heads;
     snprintf(name, sizeof(name), "%s_dq_kernel%s grid %lld x %d, %s_dkdv_kernel%s grid %lld x %d", kc.family, args,

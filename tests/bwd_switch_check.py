@@ -1,7 +1,7 @@
 """Child-process check of the 16-bit backward's forms (run by
-tests/test_bwd_forms_gpu.py with PMKL_ATTN_BWDSPLIT set; the library reads it
-once per process): the cases of test_attn_bwd_gpu.py on the form that the
-switch pins, and more of them where that form can go wrong.  Exits 0 when all
+tests/test_bwd_forms_gpu.py with PMKL_ATTN_BWDSPLIT and PMKL_ATTN_BWDWAVES set;
+the library reads them once per process): the cases of test_attn_bwd_gpu.py on the form that the
+switches pin, and more of them where that form can go wrong.  Exits 0 when all
 pass."""
 from __future__ import annotations
 
@@ -19,19 +19,20 @@ def main() -> int:
     import pmkl_amd
     from tests import test_attn_bwd_gpu as t
 
-    form = ", 2>" if os.environ["PMKL_ATTN_BWDSPLIT"] == "1" else ", 1>"
+    ks = 2 if os.environ["PMKL_ATTN_BWDSPLIT"] == "1" else 1
+    eight = ks == 1 and os.environ["PMKL_ATTN_BWDWAVES"] == "8"
     raw, launched = pmkl_amd.capi.attn_bwd_raw, set()
 
     def named(args, stream=None):   # every backward call of the cases below names its kernels first
         name = pmkl_amd.capi.attn_bwd_kernel_name(args)
-        assert name.count(form) == 2, name
+        assert name.count(f", {ks}, {8 if eight and args.head_dim == 64 else 4}>") == 2, name
         launched.add(name.split(" grid")[0])
         return raw(args, stream)
 
     pmkl_amd.capi.attn_bwd_raw = named
     dev = torch.device("cuda:0")
     for dtype in ("bf16", "fp16"):
-        for D in (32, 64, 128):
+        for D in (64,) if eight else (32, 64, 128):
             for causal in (True, False):
                 t.test_bwd_small_shapes_vs_oracle(dev, dtype, D, causal)
                 # edges of a wave's rows and of a tile, odd and even counts of tiles, more than two per workgroup
@@ -43,11 +44,12 @@ def main() -> int:
             t.test_bwd_strided_views_without_copies(dev, dtype, D)
             if D > 32:
                 t.test_bwd_with_forward_output(dev, dtype, D)
-        for causal in (True, False):
+        for causal in (True, False) if not eight else ():
             t.test_bwd_float_ml_from_64_row_kernel(dev, dtype, causal)
-    t.test_bwd_larger_heads_sampled(dev)
+    if not eight:   # head_dim 128
+        t.test_bwd_larger_heads_sampled(dev)
     t.test_bwd_closed_form_constant_v(dev)
-    assert len(launched) == 12, launched   # dtypes x head_dims x masks
+    assert len(launched) == (4 if eight else 12), launched   # dtypes x head_dims x masks
     return 0
 
 

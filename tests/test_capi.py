@@ -326,8 +326,8 @@ def test_backward_kernel_name_query():
     assert name(strides={"dq": (0, 64, 64)}) is None and "overlap" in capi.last_error()
     assert name(S=0) == "none"
     # no device, so no CU count: the 128-row form
-    assert name() == ("attn_bwd_dq_kernel<bf16, 64, causal, 1> grid 6 x 256, "
-                      "attn_bwd_dkdv_kernel<bf16, 64, causal, 1> grid 6 x 256")
+    assert name() == ("attn_bwd_dq_kernel<bf16, 64, causal, 1, 4> grid 6 x 256, "
+                      "attn_bwd_dkdv_kernel<bf16, 64, causal, 1, 4> grid 6 x 256")
     assert name(dtype=capi.PMKL_DTYPE_F32, D=128, causal=False) == (
         "attn_bwd_f32_dq_kernel<128, full> grid 20 x 256, attn_bwd_f32_dkdv_kernel<128, full> grid 20 x 256")
 
