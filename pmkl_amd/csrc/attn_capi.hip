@@ -714,13 +714,19 @@ int plan_fwd(const pmkl_attn_fwd_args *a, FwdPlan *pl) {
     const bool split = w32 && split_enabled() &&
                        (D == 64 ? causal && items < 2 * (int64_t)cu_count()
                                 : items <= (causal && S >= 1024 ? cu_count() : cu_count() / 2));
-    // fp32: 32-row workgroups whose four waves split the key tiles, at every
-    // size (measured against the 128-row kernel, us: B1 H4 S128 D64 6.3 / 17.1,
-    // B4 H16 S1024 D64 96 / 126, B2 H4 S2048 D128 144 / 326, B1 H32 S4096 D128
-    // 1,109 / 1,357, B256 H8 S20 D64 19.1 / 21.4).  The 128-row kernel is left
-    // for PMKL_ATTN_F32SPLIT=0, for a device whose CU count cannot be read, and
-    // where 32-row workgroups of 256 threads would pass a launch's 2^32 threads.
-    const bool f32split = a->dtype == PMKL_DTYPE_F32 && f32split_enabled() && cu_count() > 0 &&
+    // fp32: 32-row workgroups whose four waves split the key tiles (measured
+    // against the 128-row kernel, us: B1 H4 S128 D64 6.3 / 17.1, B4 H16 S1024 D64
+    // 96 / 126, B2 H4 S2048 D128 144 / 326, B1 H32 S4096 D128 1,109 / 1,357, B256
+    // H8 S20 D64 19.1 / 21.4).  The 128-row kernel stays the faster one where its
+    // workgroup is one full item and enough of them hide its latency: full
+    // attention over 96 to 128 keys (S128, split / 128-row: D64 512 heads 30.3 /
+    // 30.2, 768 44.0 / 41.9, 1,024 56.2 / 52.8, 4,096 233 / 190; D32 1,024 28.9 / 29.0,
+    // 1,536 41.5 / 40.3, 4,096 101 / 95; D128, causal and S <= 64 never).  It also runs with
+    // PMKL_ATTN_F32SPLIT=0, on a device whose CU count cannot be read, and where
+    // 32-row workgroups of 256 threads would pass a launch's 2^32 threads.
+    const int64_t full128 = D == 64 ? 3 : D == 32 ? 6 : 0;   // heads per CU, from
+    const bool tall = !causal && S >= 96 && S <= 128 && full128 > 0 && B * H >= full128 * (int64_t)cu_count();
+    const bool f32split = a->dtype == PMKL_DTYPE_F32 && f32split_enabled() && cu_count() > 0 && !tall &&
                           B * H * ((S + 31) / 32) < (1LL << 24);
     const KernelChoice kc = w32        ? (bf ? pick_w32<__bf16>(D, causal, split) : pick_w32<_Float16>(D, causal, split))
                             : f32split ? pick32split(D, causal)

@@ -34,3 +34,31 @@ def test_fp32_split_edges(device, D, causal):
                 continue
             got, ref, fl = _run(B, H, S, D, "fp32", causal, seed=9200 + i, with_o=with_o)
             _check(got, ref, "fp32", f"{tag} with_o={with_o}", fl)
+
+
+@pytest.mark.parametrize("D, B, H", [(64, 24, 32), (32, 48, 32)])
+def test_fp32_forward_128_row_workgroups(device, D, B, H):
+    """Full attention over 96 to 128 keys with many heads: the 128-row kernel
+    (256 CUs), at both ends of the range; the key-split kernel beside it."""
+    import torch
+
+    import pmkl_amd
+    from pmkl_amd import capi
+    from pmkl_amd.workloads import small_inputs
+    from tests.parity import check_outputs
+
+    def name(heads, S, causal=False):
+        f32 = capi.PMKL_DTYPE_F32
+        return capi.attn_fwd_kernel_name(capi.make_args(*range(0x1000, 0x7000, 0x1000), dtype=f32, batch=1, heads=heads,
+                                                        seq_len=S, head_dim=D, is_causal=causal))
+
+    for S in (96, 128):
+        assert name(B * H, S).startswith("attn_fwd_f32_kernel"), name(B * H, S)
+        tag = f"fp32 B{B} H{H} S{S} D{D} full"
+        _say(f"case {tag}")
+        q, k, v = small_inputs(B, H, S, D, "fp32", seed=9700 + S)
+        o, m, l = pmkl_amd.attn_fwd(q.to(device), k.to(device), v.to(device), is_causal=False)
+        torch.cuda.synchronize()
+        check_outputs(q, k, v, o, m, l, "fp32", causal=False, label=tag)
+    for heads, S, causal in ((B * H, 95, False), (B * H, 129, False), (B * H, 128, True), (B * H - 1, 128, False)):
+        assert name(heads, S, causal).startswith("attn_fwd_f32_split_kernel"), (heads, S, causal)
