@@ -206,7 +206,9 @@ bool f32split_enabled() {
 // rows from 1,024 on up to one item per CU, where the longest item sets the
 // time (us without / with, by items: full S2047 128: 47.8 / 41.1, 256: 68.3 /
 // 77.8; causal S512 128: 19.5 / 15.5, 256: 22.0 / 23.5; causal S2047 128: 45.3 /
-// 35.2, 256: 51.3 / 46.9; causal S1024 256: 32.3 / 30.3).
+// 35.2, 256: 51.3 / 46.9; causal S1024 256: 32.3 / 30.3; between S 1,024 and 1,280
+// the second item of a workgroup costs more than it gains from 1.5 128-row items
+// per CU on: S1200 49 heads 33.9 / 36.3).
 template <typename T>
 KernelChoice pick_w32(int64_t D, bool causal, bool split) {
     if (D == 64 && causal && split)
@@ -710,10 +712,11 @@ int plan_fwd(const pmkl_attn_fwd_args *a, FwdPlan *pl) {
     const int waves = small128 && !waves16_env() ? 4 : waves16(D, S, causal);
     const bool resident = !w64 && a->dtype != PMKL_DTYPE_F32 && waves == 8 &&
                           (S + 63) / 64 <= resident_tiles(D) && resident_enabled();
-    const int64_t items = B * H * ((S + 255) / 256);
+    const int64_t items = B * H * ((S + 255) / 256), cus = cu_count();
+    const bool long_causal = causal && S >= 1024 &&
+                             (S == 1024 || S >= 1280 || 2 * B * H * ((S + 127) / 128) <= 3 * cus);
     const bool split = w32 && split_enabled() &&
-                       (D == 64 ? causal && items < 2 * (int64_t)cu_count()
-                                : items <= (causal && S >= 1024 ? cu_count() : cu_count() / 2));
+                       (D == 64 ? causal && items < 2 * cus : items <= (long_causal ? cus : cus / 2));
     // fp32: 32-row workgroups whose four waves split the key tiles (measured
     // against the 128-row kernel, us: B1 H4 S128 D64 6.3 / 17.1, B4 H16 S1024 D64
     // 96 / 126, B2 H4 S2048 D128 144 / 326, B1 H32 S4096 D128 1,109 / 1,357, B256
@@ -762,13 +765,19 @@ int plan_fwd(const pmkl_attn_fwd_args *a, FwdPlan *pl) {
     p.lazy_raw = pmkl_amd::kLazyLog2 / p.scale_log2;   // IEEE float division, as the kernels' was
     p.ml_f32 = a->ml_dtype == PMKL_DTYPE_F32 ? 1 : 0;
     // XCD-grouped issue order needs whole head pairs (causal) or heads per XCD.
-    p.xcd_order = (a->dtype != PMKL_DTYPE_F32 && xcd_order_enabled() && (B * H) % (a->is_causal ? 16 : 8) == 0) ? 1 : 0;
+    // It issues a head pair's items longest first, then the next pair's; where a
+    // CU of the 128-row form at head_dim 128 takes a second item, its lengths even
+    // out only if an XCD's workgroups hold whole pairs (S1800 32 heads: 56.9 us, in
+    // plain order 39.2).
+    const int64_t per_xcd = cus / 8, pair = 2 * n_qtiles;
+    const bool even_pairs = !(split && D == 128 && causal) || n_qtiles * B * H <= cus || per_xcd % pair == 0;
+    p.xcd_order = (a->dtype != PMKL_DTYPE_F32 && xcd_order_enabled() && even_pairs &&
+                   (B * H) % (a->is_causal ? 16 : 8) == 0) ? 1 : 0;
 
     // One workgroup per work item, except the 64-row kernel: one workgroup per
     // CU, each looping over its share of the items.
     int64_t grid = n_qtiles * B * H;
     if (w64) {
-        const int cus = cu_count();
         PMKL_REQUIRE(cus > 0, PMKL_EHIP, "could not read the device's CU count");
         grid = std::min<int64_t>(grid, (int64_t)kc.per_cu * cus);
     }

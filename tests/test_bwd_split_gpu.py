@@ -103,3 +103,30 @@ def test_forward_small_item_count(device):
         assert "attn_fwd_w64_kernel" in pmkl_amd.capi.attn_fwd_kernel_name(args)
         assert "1, 4>" in pmkl_amd.capi.attn_fwd_kernel_name(args)
         check_outputs(q, k, v, o, m, l, dtype, causal=causal, label=tag)
+
+
+def test_forward_small_item_count_rule(device):
+    """Head_dim 128 causal: where 128-row work items and their order over the XCDs
+    are the faster (256 CUs), and the results on a plain order with two items per
+    workgroup."""
+    import torch
+
+    import pmkl_amd
+    from pmkl_amd import capi
+    from pmkl_amd.workloads import small_inputs
+    from tests.parity import check_outputs
+
+    def name(BH, S):
+        return capi.attn_fwd_kernel_name(capi.make_args(*range(0x1000, 0x7000, 0x1000), dtype=capi.PMKL_DTYPE_BF16,
+                                                        batch=1, heads=BH, seq_len=S, head_dim=128))
+
+    for BH, S, form, xcd in ((32, 1800, ", 1, 4>", False), (32, 1500, ", 1, 4>", False), (32, 2047, ", 1, 4>", True),
+                             (64, 1024, ", 1, 4>", True), (16, 1500, ", 1, 4>", True), (48, 1030, ", 1, 8>", True),
+                             (49, 1200, ", 1, 8>", False), (40, 1200, ", 1, 8>", False), (38, 1200, ", 1, 4>", False)):
+        assert form in name(BH, S) and ("xcd order" in name(BH, S)) == xcd, (BH, S, name(BH, S))
+    q, k, v = small_inputs(2, 16, 1500, 128, "bf16", seed=9450)
+    o, m, l = pmkl_amd.attn_fwd(q.to(device), k.to(device), v.to(device))
+    torch.cuda.synchronize()
+    heads = lambda t: t[:, [0, 7, 15]]
+    check_outputs(*map(heads, (q, k, v)), *(heads(t).contiguous() for t in (o, m, l)), "bf16", causal=True,
+                  label="bf16 B2 H16 S1500 D128")
