@@ -15,7 +15,8 @@
 // Bound: v_mfma_f32_32x32x2f32 (attn_f32.hpp).  Each wave stages its own
 // tiles, V then K (dout, Q, dout) through one LDS tile and one set of staging
 // registers, the next one in flight under the products of the one before: the
-// waves of a SIMD (4 / 3 / 1 at head_dim 32 / 64 / 128) drift apart and one's
+// waves of a SIMD (4 / 3 / 1 at head_dim 32 / 64 / 128; at 64 the dK/dV pass
+// spills 2-3 registers for its third) drift apart and one's
 // exponentials and LDS writes pass under the other's MFMAs.  32 owned rows and
 // a four-way split give many short, equal workgroups: the chains of dependent
 // tiles are a quarter as long as with one wave per row block, which bounds the

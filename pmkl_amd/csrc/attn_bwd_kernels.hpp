@@ -631,9 +631,9 @@ __global__ __launch_bounds__(NW * 64, D >= 128 ? 1 : 2) void attn_bwd_dkdv_kerne
     }
     const float c = p.scale_log2;
 
-    // ---- staging of Q, dout (two layouts each) and the row vectors ----
+    // ---- staging of Q, dout and the row vectors ----
     u32x4_t qreg[LOADS], oreg[LOADS];
-    float vreg;      // one row-vector element per thread (threads 0..127)
+    float vreg;      // one row-vector element per thread (threads 0 .. 2 BN - 1: lse2, then D_n)
     int goffq[LOADS], goffo[LOADS];   // lane byte offsets of its chunks in a Q / dout tile
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) {
@@ -788,7 +788,8 @@ __global__ __launch_bounds__(NW * 64, D >= 128 ? 1 : 2) void attn_bwd_dkdv_kerne
                 });
                 __builtin_amdgcn_sched_barrier(0);
             } else {
-                // Plain tile (the half-tile pipeline spills at 8 waves):
+                // Plain tile (256 registers, two waves per SIMD: the half-tile
+                // pipeline would spill; causal split form at 64: 4 spilled):
                 // S = Q K^T, dP = dout V^T: MFMA m is (dk, qb, which) = (m / 4,
                 // (m / 2) % 2, m % 2), four interleaved chains, row fragments read
                 // RING MFMAs ahead

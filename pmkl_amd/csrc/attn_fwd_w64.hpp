@@ -259,9 +259,11 @@ template <int D, int QB> struct W64Sched {
 // QB 32-row query blocks per wave, NW waves per workgroup, 32 QB NW query
 // rows per workgroup: (QB, NW) = (2, 4) is one wave of 64 rows per SIMD;
 // (1, 8) two waves of 32 rows per SIMD, each running the same slot schedule,
-// so that one wave issues while the other waits; (1, 4) the same two waves
-// per SIMD from two workgroups of 128 rows on one CU (head_dim 64: 64 KiB of
-// LDS each), which halves the work item for problems with few items.
+// so that one wave issues while the other waits; (1, 4) has 128-row workgroups,
+// which halves the work item for problems with few items.  At head_dim 64 (64 KiB
+// of LDS) two of them share a CU, the same two waves per SIMD; at head_dim 128
+// (128 KiB) one has the CU, one wave per SIMD, whatever its register bound (it
+// takes 276, without spills).
 template <typename T, int D, bool CAUSAL, int QB = 2, int NW = 4>
 __global__ __launch_bounds__(64 * NW, (QB == 1 && NW == 4) ? 2 : 1)
 __attribute__((amdgpu_waves_per_eu(QB == 1 ? 2 : NW / 4, QB == 1 ? 2 : NW / 4)))

@@ -16,9 +16,9 @@
 // Outputs are allocated contiguous [B, H, S, D] (the reference uses
 // empty_like(v), which keeps a strided v's layout while the body writes it as
 // if it were contiguous); out_m and out_l are [B, H, S] in v's dtype.
-// The backward does the same split: device tensors (fp16 / bf16) go to
-// pmkl_attn_bwd with a workspace from torch's allocator, CPU tensors to
-// host_attention_backward, the reference's per-element steps.
+// The backward does the same split: device tensors go to pmkl_attn_bwd with a
+// workspace from torch's allocator, CPU tensors to host_attention_backward, the
+// reference's per-element steps.
 #include <torch/extension.h>
 
 #include <ATen/Parallel.h>

@@ -14,8 +14,8 @@ Dispatch:
 Backward (gradients of out only; those of out_m, out_l are ignored, as in the
 reference, __init__.py:25-32): CPU with debug=True -> fused_self_attention_bw's
 CPU body, as the reference; ROCm float32 / float16 / bfloat16 tensors ->
-pmkl_attn_bwd (the gfx950 backward: vector-ALU kernels for float32, MFMA for
-the 16-bit types), given the saved forward output so its row terms come from
+pmkl_attn_bwd (the gfx950 backward, MFMA kernels; float32 on the vector ALUs for
+short sequences), given the saved forward output so its row terms come from
 <dout, out>; anything else -> NotImplementedError.
 """
 import torch
