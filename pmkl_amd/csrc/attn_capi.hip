@@ -461,14 +461,15 @@ int bwd_waves_mode() {
 //   full    S 2048  384: 120.0 / 111.5, 768: 196.6 / 233.3;  S 8192  384: 440 / 397, 512: 487 / 464, 896: 921 / 857,
 //           1024: 953 / 926, 1280: 1,190 / 1,309, 1536: 1,414 / 1,378;  S 1024  288: 65.5 / 63.0, 512: 75.3 / 81.6
 //           (without O  320: 78.7 / 82.4)
-//   causal  S 8192  1024: 542 / 504, 768: 411 / 447, 512: 335 / 411;  S 2048  1024: 154.5 / 151.8, 640: 104 / 118
+//   causal  S 8192  1024: 542 / 504, 768: 411 / 447, 512: 335 / 411 (without O  832: 575 / 594);  S 2048  1024:
+//           154.5 / 151.8, 640: 104 / 118
 bool bwd_eight(const pmkl_attn_bwd_args *a, bool split) {
     const int64_t S = a->seq_len, cus = cu_count();
     if (split || a->head_dim != 64) return false;
     if (bwd_waves_mode() != 0) return bwd_waves_mode() == 8;
     if (cus <= 0 || S < 768) return false;
     const int64_t groups = a->batch * a->heads * ((S + 127) / 128), share = (groups + cus - 1) / cus;
-    if (a->is_causal != 0) return S >= 4096 && share == 4;
+    if (a->is_causal != 0) return S >= 4096 && share == 4 && (a->o != nullptr || 4 * groups > 13 * cus);
     if (S < 1536) return share == 2 && a->o != nullptr && groups <= 7 * cus / 4;
     return share == 2 || (S >= 4096 && (share == 4 || share == 6));
 }

@@ -45,6 +45,7 @@ def test_backward_form_rule(device):
                           (12, 8192, True), (64, 2048, True), (24, 8192, True), (64, 8192, False)):
         assert form(BH, S, 64, causal) == (1, 4), (BH, S, causal)
     assert form(36, 1024, 64, False) == (1, 8) and form(36, 1024, 64, False, with_o=False) == (1, 4)
+    assert form(26, 4096, 64, True) == (1, 8) and form(26, 4096, 64, True, with_o=False) == (1, 4)
     assert form(24, 2047, 32, False) == form(24, 2047, 128, False) == (1, 4)
 
 
