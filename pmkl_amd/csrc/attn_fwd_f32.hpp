@@ -101,7 +101,8 @@ __global__ __launch_bounds__(kF32Threads, D >= 128 ? 2 : D >= 64 ? 3 : 4) void a
 
     // O = sum_w 2^((m_w - M) c) O_w / l over the waves, M = max_w m_w and l the
     // sum of theirs likewise: each wave scales its own O, the scaled ones are
-    // added.  A wave without tiles holds m = -inf and weighs 0.
+    // added.  A wave without tiles holds m = -inf and weighs 0; a row of -inf
+    // scores alone has M = -inf, and l and O NaN as in the reference.
     const float l_w = half_sum(l_run);
     if (hi == 0) {
         mlvec[wave][0][col] = m_run;
@@ -111,10 +112,9 @@ __global__ __launch_bounds__(kF32Threads, D >= 128 ? 2 : D >= 64 ? 3 : 4) void a
     float M = -INFINITY, l_tot = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) M = fmaxf(M, mlvec[w][0][col]);
-    const float Mu = M == -INFINITY ? 0.f : M;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) l_tot += fast_exp2((mlvec[w][0][col] - Mu) * c) * mlvec[w][1][col];
-    const float f = fast_exp2((m_run - Mu) * c) * (1.0f / l_tot);
+    for (int w = 0; w < NW; ++w) l_tot += fast_exp2((mlvec[w][0][col] - M) * c) * mlvec[w][1][col];
+    const float f = fast_exp2((m_run - M) * c) * (1.0f / l_tot);
     if (wave < nt) {
 #pragma unroll
         for (int db = 0; db < NDB; ++db) acc[db] *= f;

@@ -83,3 +83,28 @@ def test_fp32_backward_nonfinite_rows(device, D, causal):
                         assert np.array_equal(g[~fin], w[~fin], equal_nan=True), f"{tag}: {grad} not finite elsewhere"
                         err = np.abs(g - w)[fin]
                         assert (err <= TOL["fp32"] * max(fl, 1.0)).all(), f"{tag}: {grad} off by {err.max()}"
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_fp32_forward_row_of_minus_infinities(device, D):
+    """The first query sees one key, whose score is -inf: m = -inf and l, o NaN,
+    as the sums of exp(-inf - -inf) are; the other rows give that key no weight."""
+    import torch
+
+    import pmkl_amd
+
+    for H, S in ((2, 77), (2, 290), (600, 130)):
+        rng = np.random.Generator(np.random.PCG64(S + D))
+        q, k, v = (rng.standard_normal((H, S, D)).astype(np.float32).astype(np.float64) for _ in range(3))
+        q = np.abs(q)
+        k[:, 0] = -INF
+        with np.errstate(all="ignore"):
+            want = _forward(q[:2], k[:2], v[:2], True)
+        got = pmkl_amd.attn_fwd(*(torch.from_numpy(x.astype(np.float32)).to(device)[None] for x in (q, k, v)))
+        torch.cuda.synchronize()
+        for g, w, name in zip(got, want, ("o", "m", "l")):
+            g = g[0, :2].cpu().numpy().astype(np.float64)
+            fin = np.isfinite(w)
+            assert fin.any() and not fin.all()
+            assert np.array_equal(g[~fin], w[~fin], equal_nan=True), f"H{H} S{S} D{D}: {name} not finite elsewhere"
+            assert (np.abs(g - w)[fin] <= 1e-5 * np.abs(w[fin]).max()).all(), f"H{H} S{S} D{D}: {name}"
