@@ -394,13 +394,13 @@ BwdKernels pick_bwd_f32(bool causal, bool rows) {
 // heads D 64 213 / 138;  S 8  128 heads D 64 16.9 / 11.9, D 128 27.7 / 20.0;  S 16
 // 16 heads D 64 17.0 / 13.0;  S 31  16 heads D 128 28.0 / 25.9.  The lines lie
 // where the two meet, by the rows' workgroups (4 rows) per CU: up to S 6 (head_dim
-// 128: 8) rows at any count, then while few of them queue.  A launch's 2^32
+// 128: 7) rows at any count, then while few of them queue.  A launch's 2^32
 // threads are 2^26 rows here and 2^24 heads there.
 bool bwd_f32_rows(const pmkl_attn_bwd_args *a) {
     const int64_t S = a->seq_len, D = a->head_dim, rows = a->batch * a->heads * S;
     if (rows >= (1LL << 26)) return false;
-    if (S <= (D == 128 ? 8 : 6)) return true;
-    const int64_t per_cu = D == 128  ? (S <= 36 ? 1 : 0)
+    if (S <= (D == 128 ? 7 : 6)) return true;
+    const int64_t per_cu = D == 128  ? (S <= 8 ? 3 : S <= 36 ? 1 : 0)
                            : D == 64 ? (S <= 8 ? 3 : S <= 14 ? 2 : S <= (a->is_causal ? 36 : 28) ? 1 : 0)
                                      : (S <= 8 ? 2 : S <= 14 ? 1 : 0);
     return rows <= pmkl_amd::kF32RowWaves * per_cu * cu_count();

@@ -22,9 +22,9 @@ def _name(BH, S, D, causal=True):
 def test_fp32_backward_rows_or_tiles(device):
     # (heads, S, head_dim): rows where they are the faster, on a device of 256 CUs
     for BH, S, D in ((1, 1, 32), (65536, 4, 32), (256, 8, 32), (64, 14, 32), (8192, 6, 64), (384, 8, 64), (128, 14, 64),
-                     (32, 28, 64), (16, 33, 64), (65536, 8, 128), (64, 16, 128), (16, 36, 128)):
+                     (32, 28, 64), (16, 33, 64), (65536, 7, 128), (384, 8, 128), (64, 16, 128), (16, 36, 128)):
         assert "attn_bwd_f32_row_dq_kernel" in _name(BH, S, D), (BH, S, D)
-    for BH, S, D in ((1024, 8, 32), (1, 16, 32), (1024, 8, 64), (192, 14, 64), (64, 24, 64), (1, 37, 64), (128, 16, 128),
+    for BH, S, D in ((1024, 8, 32), (1, 16, 32), (1024, 8, 64), (1024, 8, 128), (192, 14, 64), (64, 24, 64), (1, 37, 64), (128, 16, 128),
                      (1, 48, 128)):
         assert "attn_bwd_f32_dq_kernel" in _name(BH, S, D), (BH, S, D)
 
